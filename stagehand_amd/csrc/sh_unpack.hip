@@ -14,13 +14,14 @@
 // each workgroup its descriptor in O(1) (one scalar load), and the descriptor
 // itself is a 64-byte scalar load, so all per-region state lives in SGPRs.
 // Each thread moves `unroll` chunks; all loads of a thread are issued before
-// the first conversion. Loads and stores are up to 128-bit (an int8 chunk of
-// 8 is a 64-bit load and a 128-bit bf16 store; the cast reads 128 and writes
-// 64 bits); the hardware's unaligned-access mode lets them start at any byte
-// offset, which the reference layout needs (it has no padding, so int8 regions
-// start at arbitrary offsets). With int8 chunks of 8, every chunk of a row
-// whose length is a multiple of 8 needs one row scale, loaded once per chunk;
-// shorter or ragged rows take an element-wise path. This is pure
+// the first conversion. Loads and stores are up to 128-bit (an int8 chunk is
+// one 128-bit store: 8 values to bf16 from a 64-bit load, 4 to fp32 from a
+// 32-bit load; the cast reads 128 and writes 64 bits); the hardware's
+// unaligned-access mode lets them start at any byte offset, which the reference
+// layout needs (it has no padding, so int8 regions start at arbitrary offsets).
+// A chunk inside one row needs one row scale; a chunk across two rows takes a
+// second one and, from a padded source, a second load. Only rows shorter than a
+// chunk and chunks cut by a region's ends go element by element. This is pure
 // streaming: no LDS (the scale is one load per chunk) and no MFMA.
 //
 // Numerics. The dequant is computed exactly as the reference's torch CPU ops:
@@ -134,33 +135,28 @@ __device__ __forceinline__ float dq(float q, float s, float z) {
 
 // ── INT8 row-scale dequant ────────────────────────────────────────────────
 
-// One chunk of C int8 values of a single row → C outputs.
-template <uint32_t C, bool OUT_BF16, bool HAS_ZP, bool NANCHK>
-__device__ __forceinline__ void dq_chunk_store(const Words<C>& q, float s, float z, uint8_t* out) {
-  if (OUT_BF16) {
-    Words<2 * C> o;
+// One chunk of C int8 values of a single row with a finite scale and zero point (they cannot turn
+// a finite q into NaN) → C outputs.
+template <uint32_t C, bool OUT_BF16, bool HAS_ZP>
+__device__ __forceinline__ Words<C * (OUT_BF16 ? 2 : 4)> dq_chunk(const Words<C>& q, float s, float z) {
+  Words<C * (OUT_BF16 ? 2 : 4)> o;
+  if constexpr (OUT_BF16) {
 #pragma unroll
-    for (uint32_t w = 0; w < C / 4; ++w) {
-      const uint32_t word = q.w[w];
-      const float f0 = dq<HAS_ZP>(i8_at(word, 0), s, z);
-      const float f1 = dq<HAS_ZP>(i8_at(word, 1), s, z);
-      const float f2 = dq<HAS_ZP>(i8_at(word, 2), s, z);
-      const float f3 = dq<HAS_ZP>(i8_at(word, 3), s, z);
-      o.w[2 * w] = NANCHK ? pack_hi(rne_hi_nan(f0), rne_hi_nan(f1)) : pack_hi(rne_hi(f0), rne_hi(f1));
-      o.w[2 * w + 1] = NANCHK ? pack_hi(rne_hi_nan(f2), rne_hi_nan(f3)) : pack_hi(rne_hi(f2), rne_hi(f3));
+    for (uint32_t w = 0; w < C / 2; ++w) {
+      const uint32_t word = q.w[w / 2];
+      o.w[w] = pack_hi(rne_hi(dq<HAS_ZP>(i8_at(word, (2 * w) % 4), s, z)),
+                       rne_hi(dq<HAS_ZP>(i8_at(word, (2 * w + 1) % 4), s, z)));
     }
-    stw_nt<2 * C>(out, o);  // written once, read by the next kernel: no reason to keep it in L2
   } else {
-    Words<4 * C> o;
 #pragma unroll
     for (uint32_t j = 0; j < C; ++j) o.w[j] = __float_as_uint(dq<HAS_ZP>(i8_at(q.w[j / 4], j % 4), s, z));
-    stw<4 * C>(out, o);
   }
+  return o;
 }
 
 template <bool OUT_BF16>
 __device__ __forceinline__ void store_elem(uint8_t* o, uint32_t idx, float v) {
-  if (OUT_BF16) {
+  if constexpr (OUT_BF16) {
     const uint16_t b = bf16_bits(v);
     __builtin_memcpy(o + 2 * (size_t)idx, &b, 2);
   } else {
@@ -168,106 +164,209 @@ __device__ __forceinline__ void store_elem(uint8_t* o, uint32_t idx, float v) {
   }
 }
 
-template <bool OUT_BF16, bool HAS_ZP>
-__device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
-                                        const uint8_t* __restrict__ src,
-                                        const float* __restrict__ scales,
-                                        const float* __restrict__ zps, uint8_t* __restrict__ dst) {
-  constexpr uint32_t C = kChunkI8;
-  constexpr uint32_t U = kUnrollI8;
-  constexpr uint32_t kOutBytes = OUT_BF16 ? 2 : 4;
-  const uint32_t cols = d.cols;
-  const uint32_t numel = d.rows * cols;
-  const uint32_t ld = d.src_ld ? d.src_ld : cols;
-  const uint8_t* s = src + d.src_off;
-  uint8_t* o = dst + d.dst_off;
-  const float* sc = scales + d.scale_off;
-  const float* zp = HAS_ZP ? zps + d.scale_off : nullptr;
-  // d.lead elements precede element 0 in the first tile; a chunk before the region wraps to an
-  // index >= 2^32 - 64, above every numel, and is skipped by the bounds checks below
-  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;
-
-  if (ld == cols && (cols % C) == 0) {
-    // Every chunk lies inside one row: one scale per chunk.
-    Words<C> q[U];
-    float sv[U], zv[U];
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-      const uint32_t e = e0 + k * (kThreads * C);
-      if (e < numel) q[k] = ldw<C>(s + e);
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-      const uint32_t e = e0 + k * (kThreads * C);
-      if (e < numel) {
-        const uint32_t r = sh::udiv(e, d.div_magic);
-        sv[k] = sc[r];
-        zv[k] = HAS_ZP ? zp[r] : 0.0f;
-      }
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-      const uint32_t e = e0 + k * (kThreads * C);
-      if (e < numel) {
-        uint8_t* out = o + (size_t)e * kOutBytes;
-        // A finite scale and zero point cannot turn a finite q into NaN.
-        if (__builtin_isfinite(sv[k]) && (!HAS_ZP || __builtin_isfinite(zv[k])))
-          dq_chunk_store<C, OUT_BF16, HAS_ZP, false>(q[k], sv[k], zv[k], out);
-        else
-          dq_chunk_store<C, OUT_BF16, HAS_ZP, true>(q[k], sv[k], zv[k], out);
-      }
-    }
-    return;
+// Chunk [e, e + C) of a region, element by element: a chunk cut by the region's start (e wrapped
+// below 0, so its first elements are above every numel) or end.
+template <uint32_t C, bool OUT_BF16, bool HAS_ZP>
+__device__ __forceinline__ void dq_edge(const sh_unpack_desc& d, uint32_t e, uint32_t numel, uint32_t pad,
+                                        const uint8_t* s, const float* sc, const float* zp, uint8_t* o) {
+#pragma unroll 1
+  for (uint32_t j = 0; j < C; ++j) {
+    const uint32_t i = e + j;
+    if (i >= numel) continue;
+    const uint32_t r = sh::udiv(i, d.div_magic);
+    const float q = (float)(int32_t)(int8_t)s[i + (uint64_t)r * pad];
+    store_elem<OUT_BF16>(o, i, dq<HAS_ZP>(q, sc[r], HAS_ZP ? zp[r] : 0.0f));
   }
+}
 
-  // Rows that are not a multiple of the chunk, or a padded source (ld > cols):
-  // element-wise, with the row tracked incrementally inside each chunk.
+// C outputs from the bytes of q, each with its own scale and zero point.
+template <uint32_t C, bool OUT_BF16, bool HAS_ZP>
+__device__ __forceinline__ void dq_each_store(const Words<C>& q, const float (&sv)[C], const float (&zv)[C],
+                                              uint8_t* out) {
+  if constexpr (OUT_BF16) {
+    Words<2 * C> ow;
+#pragma unroll
+    for (uint32_t w = 0; w < C / 2; ++w) {
+      const float lo = dq<HAS_ZP>(i8_at(q.w[w / 2], (2 * w) % 4), sv[2 * w], zv[2 * w]);
+      const float hi = dq<HAS_ZP>(i8_at(q.w[w / 2], (2 * w + 1) % 4), sv[2 * w + 1], zv[2 * w + 1]);
+      ow.w[w] = pack_hi(rne_hi_nan(lo), rne_hi_nan(hi));
+    }
+    stw_nt<2 * C>(out, ow);
+  } else {
+    Words<4 * C> ow;
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) ow.w[j] = __float_as_uint(dq<HAS_ZP>(i8_at(q.w[j / 4], j % 4), sv[j], zv[j]));
+    stw_nt<4 * C>(out, ow);
+  }
+}
+
+// Whether the chunk of C elements at e lies inside the region. e wraps below 0 where a lead precedes
+// element 0: to an index >= 2^32 - 4096, above every numel.
+template <uint32_t C>
+__device__ __forceinline__ bool whole_chunk(uint32_t e, uint32_t numel) {
+  return e < numel && numel - e >= C;
+}
+
+// s_waitcnt operand: every vector memory operation done, no wait for the other counters.
+constexpr int kWaitVmcnt0 = 0x0F70;
+
+// Rows of at least a chunk, of any length and stride: a chunk lies in one row, or in the last `left`
+// elements of one row and the first C - left of the next.
+//
+// All chunks of a thread go through straight-line code as if each lay in one row with a finite
+// scale: the loads first, then the conversions and the stores. Only then are the exceptions seen
+// to, which few wavefronts have: a chunk across two rows, or under a scale or zero point that can
+// make NaNs, is written once more (one wavefront's stores to one address land in program order),
+// and a chunk cut by the region's start or end is written element by element. A lane without a
+// whole chunk loads the region's first one, so that no load needs a branch; with the loads in
+// branches of their own, the compiler put waits between them for registers that other paths of the
+// kernel might have had in flight (the mixed kernel then took 172 us for a double-stream block of
+// the 12B model, and 159 after an unrelated change).
+//
+// A chunk across rows takes the second row's bytes from the same load, or in a padded source from
+// a load `pad` bytes later, whose bytes from `left` on are the next row's. Every load stays inside
+// the region: the second row exists, as the whole chunk lies below numel.
+//
+// HBM bounds this. Measured (MI355X; before, rows that were not back to back or not whole chunks
+// went element by element): a padded single-stream block of the 12B model with zero points 263 ->
+// 68 us (6.2 TB/s); 2999-wide rows 75 -> 66 us (6.1 TB/s) and a slab of 128 such tensors 1376 ->
+// 1064; the aligned double-stream block 159 -> 155 us (6.6 TB/s) and slab of 128 tensors 1011 -> 1001
+// us (6.6 TB/s).
+//
+// ALONE: the kernel holds no other kind. Once a thread has all its loads, its stores go out back to
+// back, except for aligned rows in the kernel that holds no other kind: there each store waits for
+// the one before it. Measured, not paced against paced: double-stream block (mixed kernel) 154.9
+// against 157.5 us, padded block 68.1 against 70.3; but slab of 128 aligned tensors 1030-1060 against
+// 998-1007 us (6.6 GB, and 3% from 3 GB on; up to 2 GB the same). Pacing holds back writes in a stream that is two thirds writes; why only the aligned
+// long stream gains from it is not known.
+template <bool OUT_BF16, bool HAS_ZP, bool ALONE, uint32_t C, uint32_t U>
+__device__ __forceinline__ void i8_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel, uint32_t pad,
+                                        const uint8_t* __restrict__ s, const float* __restrict__ sc,
+                                        const float* __restrict__ zp, uint8_t* __restrict__ o) {
+  constexpr uint32_t kOutBytes = OUT_BF16 ? 2 : 4;
+  Words<C> q[U];
+  float sv[U], zv[U];
+  uint32_t row[U];
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    const uint32_t e = e0 + k * (kThreads * C);
+    const uint32_t i = whole_chunk<C>(e, numel) ? e : 0u;
+    row[k] = sh::udiv(i, d.div_magic);
+    q[k] = ldw<C>(s + i + (uint64_t)row[k] * pad);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    sv[k] = sc[row[k]];
+    zv[k] = HAS_ZP ? zp[row[k]] : 0.0f;
+  }
+  if (ALONE && pad == 0 && (d.cols % C) == 0 && (d.lead % C) == 0) {
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      const uint32_t e = e0 + k * (kThreads * C);
+      const auto out = dq_chunk<C, OUT_BF16, HAS_ZP>(q[k], sv[k], zv[k]);
+      if (whole_chunk<C>(e, numel)) stw_nt<C * kOutBytes>(o + (size_t)e * kOutBytes, out);
+      if (k + 1 < U) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    }
+  } else {
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      const uint32_t e = e0 + k * (kThreads * C);
+      const auto out = dq_chunk<C, OUT_BF16, HAS_ZP>(q[k], sv[k], zv[k]);
+      if (whole_chunk<C>(e, numel)) stw_nt<C * kOutBytes>(o + (size_t)e * kOutBytes, out);
+    }
+    asm volatile("; not paced");  // keeps this tail apart from the other's, which waits in between
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    const uint32_t e = e0 + k * (kThreads * C);
+    if (!whole_chunk<C>(e, numel)) {
+      dq_edge<C, OUT_BF16, HAS_ZP>(d, e, numel, pad, s, sc, zp, o);
+      continue;
+    }
+    const uint32_t left = (row[k] + 1) * d.cols - e;  // modulo 2^32; the difference fits
+    const bool finite = !OUT_BF16 || (__builtin_isfinite(sv[k]) && (!HAS_ZP || __builtin_isfinite(zv[k])));
+    if (left >= C && finite) continue;
+    float s1 = sv[k], z1 = zv[k];
+    Words<C> qq = q[k];
+    if (left < C) {
+      s1 = sc[row[k] + 1];
+      z1 = HAS_ZP ? zp[row[k] + 1] : 0.0f;
+      if (pad != 0) {
+        const Words<C> q1 = ldw<C>(s + e + (uint64_t)row[k] * pad + pad);
+#pragma unroll
+        for (uint32_t w = 0; w < C / 4; ++w) {
+          const uint32_t own = left > 4 * w ? left - 4 * w : 0u;  // bytes of this word in the first row
+          const uint32_t m = own >= 4 ? 0xFFFFFFFFu : (1u << (8 * own)) - 1u;
+          qq.w[w] = (qq.w[w] & m) | (q1.w[w] & ~m);
+        }
+      }
+    }
+    float se[C], ze[C];
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) {
+      se[j] = j < left ? sv[k] : s1;
+      ze[j] = j < left ? zv[k] : z1;
+    }
+    dq_each_store<C, OUT_BF16, HAS_ZP>(qq, se, ze, o + (size_t)e * kOutBytes);
+  }
+}
+
+// Rows shorter than a chunk: the row is tracked element by element inside each chunk.
+template <bool OUT_BF16, bool HAS_ZP, uint32_t C, uint32_t U>
+__device__ __forceinline__ void i8_short_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel, uint32_t pad,
+                                              const uint8_t* __restrict__ s, const float* __restrict__ sc,
+                                              const float* __restrict__ zp, uint8_t* __restrict__ o) {
 #pragma unroll 1
   for (uint32_t k = 0; k < U; ++k) {
     const uint32_t e = e0 + k * (kThreads * C);
-    if (e >= numel) continue;
-    uint32_t r = sh::udiv(e, d.div_magic);
-    uint32_t c = e - r * cols;
-    const uint32_t n = min(C, numel - e);
-    if (ld == cols && n == C) {
-      const Words<C> q = ldw<C>(s + e);
-      if (OUT_BF16) {
-        uint32_t hw[C];
+    if (whole_chunk<C>(e, numel)) {
+      uint32_t r = sh::udiv(e, d.div_magic);
+      uint32_t c = e - r * d.cols;
+      Words<C> q{};
+      if (pad == 0) q = ldw<C>(s + e);
+      float se[C], ze[C];
 #pragma unroll
-        for (uint32_t j = 0; j < C; ++j) {
-          hw[j] = rne_hi_nan(dq<HAS_ZP>(i8_at(q.w[j / 4], j % 4), sc[r], HAS_ZP ? zp[r] : 0.0f));
-          if (++c == cols) {
-            c = 0;
-            ++r;
-          }
-        }
-        Words<2 * C> ow;
-#pragma unroll
-        for (uint32_t w = 0; w < C / 2; ++w) ow.w[w] = pack_hi(hw[2 * w], hw[2 * w + 1]);
-        stw<2 * C>(o + (size_t)e * 2, ow);
-      } else {
-        Words<4 * C> ow;
-#pragma unroll
-        for (uint32_t j = 0; j < C; ++j) {
-          ow.w[j] = __float_as_uint(dq<HAS_ZP>(i8_at(q.w[j / 4], j % 4), sc[r], HAS_ZP ? zp[r] : 0.0f));
-          if (++c == cols) {
-            c = 0;
-            ++r;
-          }
-        }
-        stw<4 * C>(o + (size_t)e * 4, ow);
-      }
-    } else {
-      for (uint32_t j = 0; j < n; ++j) {
-        const float q = (float)(int32_t)(int8_t)s[(size_t)r * ld + c];
-        store_elem<OUT_BF16>(o, e + j, dq<HAS_ZP>(q, sc[r], HAS_ZP ? zp[r] : 0.0f));
-        if (++c == cols) {
+      for (uint32_t j = 0; j < C; ++j) {
+        if (pad != 0) q.w[j / 4] |= (uint32_t)s[e + j + (uint64_t)r * pad] << (8 * (j % 4));
+        se[j] = sc[r];
+        ze[j] = HAS_ZP ? zp[r] : 0.0f;
+        if (++c == d.cols) {
           c = 0;
           ++r;
         }
       }
+      dq_each_store<C, OUT_BF16, HAS_ZP>(q, se, ze, o + (size_t)e * (OUT_BF16 ? 2 : 4));
+    } else {
+      dq_edge<C, OUT_BF16, HAS_ZP>(d, e, numel, pad, s, sc, zp, o);
     }
   }
+}
+
+template <bool OUT_BF16, bool HAS_ZP, bool ALONE>
+__device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
+                                        const uint8_t* __restrict__ src,
+                                        const float* __restrict__ scales,
+                                        const float* __restrict__ zps, uint8_t* __restrict__ dst) {
+  // A chunk is one 16-byte store, 8 bf16 or 4 fp32 outputs, so a wavefront's store instruction
+  // covers one contiguous 1 KiB span. With 8 fp32 per chunk each lane wrote two 16-byte halves at a
+  // 32-byte stride: a float32 double-stream block (hidden 1536) 84 us, now 62 (6.9 TB/s); plain
+  // instead of non-temporal fp32 stores 76 us.
+  constexpr uint32_t C = OUT_BF16 ? kChunkI8 : kStepI8F32;
+  constexpr uint32_t U = kUnrollI8 * kChunkI8 / C;
+  constexpr uint32_t T = kThreads * U * C;
+  const uint32_t cols = d.cols;
+  const uint32_t numel = d.rows * cols;
+  const uint32_t pad = d.src_ld - cols;  // src_ld is never 0 in a launch table
+  const uint8_t* s = src + d.src_off;
+  uint8_t* o = dst + d.dst_off;
+  const float* sc = scales + d.scale_off;
+  const float* zp = HAS_ZP ? zps + d.scale_off : nullptr;
+  const uint32_t e0 = local * T + threadIdx.x * C - d.lead;
+  if (cols >= C)
+    i8_rows<OUT_BF16, HAS_ZP, ALONE, C, U>(d, e0, numel, pad, s, sc, zp, o);
+  else
+    i8_short_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, pad, s, sc, zp, o);
 }
 
 // ── fp32 → bf16 cast ──────────────────────────────────────────────────────
@@ -280,24 +379,26 @@ __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t 
   const uint32_t numel = d.rows * d.cols;
   const uint8_t* s = src + d.src_off;
   uint8_t* o = dst + d.dst_off;
-  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;  // wraps before the region
+  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;
   Words<4 * C> v[U];
 #pragma unroll
   for (uint32_t k = 0; k < U; ++k) {
     const uint32_t e = e0 + k * (kThreads * C);
-    if (e < numel && numel - e >= C) v[k] = ldw_nt<4 * C>(s + (size_t)e * 4);  // read once
+    if (whole_chunk<C>(e, numel)) v[k] = ldw_nt<4 * C>(s + (size_t)e * 4);  // read once
   }
 #pragma unroll
   for (uint32_t k = 0; k < U; ++k) {
     const uint32_t e = e0 + k * (kThreads * C);
-    if (e < numel && numel - e >= C) {
+    if (whole_chunk<C>(e, numel)) {
       Words<2 * C> ow;
 #pragma unroll
       for (uint32_t w = 0; w < C / 2; ++w)
         ow.w[w] = pack_hi(rne_hi_nan(__uint_as_float(v[k].w[2 * w])), rne_hi_nan(__uint_as_float(v[k].w[2 * w + 1])));
       stw<2 * C>(o + (size_t)e * 2, ow);
-    } else if (e < numel) {
-      for (uint32_t j = e; j < numel; ++j) {
+    } else {
+#pragma unroll 1
+      for (uint32_t j = e; j != e + C; ++j) {  // cut by the region's start or end
+        if (j >= numel) continue;
         float x;
         __builtin_memcpy(&x, s + (size_t)j * 4, 4);
         const uint16_t b = bf16_bits(x);
@@ -309,34 +410,39 @@ __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t 
 
 // ── bf16 → fp32 widen ─────────────────────────────────────────────────────
 
+// A tile is kThreads * kChunkB16 elements, moved kStepB16 at a time (one 16-byte store) with
+// consecutive lanes on consecutive steps, so each store instruction of a wavefront covers one
+// contiguous 1 KiB span.
 __device__ __forceinline__ void tile_bf16_f32(const sh_unpack_desc& d, uint32_t local,
                                               const uint8_t* __restrict__ src,
                                               uint8_t* __restrict__ dst) {
-  constexpr uint32_t C = kChunkB16;
-  constexpr uint32_t U = 1;
+  constexpr uint32_t C = kStepB16;
+  constexpr uint32_t U = kChunkB16 / kStepB16;
   const uint32_t numel = d.rows * d.cols;
   const uint8_t* s = src + d.src_off;
   uint8_t* o = dst + d.dst_off;
-  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;  // wraps before the region
+  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;
   Words<2 * C> v[U];
 #pragma unroll
   for (uint32_t k = 0; k < U; ++k) {
     const uint32_t e = e0 + k * (kThreads * C);
-    if (e < numel && numel - e >= C) v[k] = ldw<2 * C>(s + (size_t)e * 2);
+    if (whole_chunk<C>(e, numel)) v[k] = ldw<2 * C>(s + (size_t)e * 2);
   }
 #pragma unroll
   for (uint32_t k = 0; k < U; ++k) {
     const uint32_t e = e0 + k * (kThreads * C);
-    if (e < numel && numel - e >= C) {
+    if (whole_chunk<C>(e, numel)) {
       Words<4 * C> ow;
 #pragma unroll
       for (uint32_t w = 0; w < C / 2; ++w) {
         ow.w[2 * w] = v[k].w[w] << 16;
         ow.w[2 * w + 1] = v[k].w[w] & 0xFFFF0000u;
       }
-      stw<4 * C>(o + (size_t)e * 4, ow);
-    } else if (e < numel) {
-      for (uint32_t j = e; j < numel; ++j) {
+      stw_nt<4 * C>(o + (size_t)e * 4, ow);
+    } else {
+#pragma unroll 1
+      for (uint32_t j = e; j != e + C; ++j) {  // cut by the region's start or end
+        if (j >= numel) continue;
         uint16_t b;
         __builtin_memcpy(&b, s + (size_t)j * 2, 2);
         const uint32_t w = (uint32_t)b << 16;
@@ -348,26 +454,23 @@ __device__ __forceinline__ void tile_bf16_f32(const sh_unpack_desc& d, uint32_t 
 
 // ── byte copy / zero fill ─────────────────────────────────────────────────
 
+// A tile is kThreads * C bytes, moved as 16-byte words with consecutive lanes on consecutive words
+// (each load / store instruction of a wavefront covers one contiguous 1 KiB span).
 template <bool ZERO>
 __device__ __forceinline__ void tile_bytes(const sh_unpack_desc& d, uint32_t local,
                                            const uint8_t* __restrict__ src,
                                            uint8_t* __restrict__ dst) {
-  // A tile is kThreads * U * C bytes, moved as 16-byte words with
-  // consecutive lanes on consecutive words (each load / store instruction of a
-  // wavefront covers one contiguous 1 KiB span).
-  constexpr uint32_t C = ZERO ? kChunkZero : kChunkCopy;
-  constexpr uint32_t U = 1;
   constexpr uint32_t W = 16;
-  constexpr uint32_t kWords = U * (C / W);
+  constexpr uint32_t kWords = (ZERO ? kChunkZero : kChunkCopy) / W;
   const uint32_t nbytes = d.rows * d.cols;
   const uint8_t* s = src + d.src_off;
   uint8_t* o = dst + d.dst_off;
-  const uint32_t t0 = local * (kThreads * U * C) - d.lead;  // wraps before the region
+  const uint32_t b0 = local * (kThreads * kWords * W) + threadIdx.x * W - d.lead;
   Words<W> v[kWords];
 #pragma unroll
   for (uint32_t k = 0; k < kWords; ++k) {
-    const uint32_t b = t0 + (k * kThreads + threadIdx.x) * W;
-    if (b < nbytes && nbytes - b >= W) {
+    const uint32_t b = b0 + k * (kThreads * W);
+    if (whole_chunk<W>(b, nbytes)) {
       if (ZERO) {
 #pragma unroll
         for (uint32_t w = 0; w < W / 4; ++w) v[k].w[w] = 0;
@@ -378,11 +481,13 @@ __device__ __forceinline__ void tile_bytes(const sh_unpack_desc& d, uint32_t loc
   }
 #pragma unroll
   for (uint32_t k = 0; k < kWords; ++k) {
-    const uint32_t b = t0 + (k * kThreads + threadIdx.x) * W;
-    if (b < nbytes && nbytes - b >= W) {
+    const uint32_t b = b0 + k * (kThreads * W);
+    if (whole_chunk<W>(b, nbytes)) {
       stw<W>(o + b, v[k]);
-    } else if (b < nbytes) {
-      for (uint32_t j = b; j < nbytes; ++j) o[j] = ZERO ? (uint8_t)0 : s[j];
+    } else {
+#pragma unroll 1
+      for (uint32_t j = b; j != b + W; ++j)  // cut by the region's start or end
+        if (j < nbytes) o[j] = ZERO ? (uint8_t)0 : s[j];
     }
   }
 }
@@ -416,7 +521,7 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
   // The single-kind kernels are launched only for plans whose every descriptor has that kind
   // (launch_tiles), so they test no kind.
   if constexpr (MASK == kMaskDequantBf16) {
-    tile_i8<true, HAS_ZP>(d, local, src, scales, zps, dst);
+    tile_i8<true, HAS_ZP, true>(d, local, src, scales, zps, dst);
     return;
   }
   if constexpr (MASK == kMaskCastBf16) {
@@ -426,11 +531,11 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
   switch (d.kind) {
     case SH_KIND_I8_ROWSCALE_BF16:
       if constexpr ((MASK & bit(SH_KIND_I8_ROWSCALE_BF16)) != 0)
-        tile_i8<true, HAS_ZP>(d, local, src, scales, zps, dst);
+        tile_i8<true, HAS_ZP, false>(d, local, src, scales, zps, dst);
       break;
     case SH_KIND_I8_ROWSCALE_F32:
       if constexpr ((MASK & bit(SH_KIND_I8_ROWSCALE_F32)) != 0)
-        tile_i8<false, HAS_ZP>(d, local, src, scales, zps, dst);
+        tile_i8<false, HAS_ZP, false>(d, local, src, scales, zps, dst);
       break;
     case SH_KIND_F32_BF16:
       if constexpr ((MASK & bit(SH_KIND_F32_BF16)) != 0) tile_f32_bf16(d, local, src, dst);

@@ -42,8 +42,12 @@ constexpr uint32_t kThreads = SH_UNPACK_THREADS;
 constexpr uint32_t kUnrollI8 = SH_UNROLL_I8;
 constexpr uint32_t kUnrollF32 = SH_UNROLL_F32;
 constexpr uint32_t kChunkI8 = SH_CHUNK_I8;     // int8 elements per thread per chunk
+// Elements per 16-byte fp32 store: the dequant to fp32 and the widen move their tile in such steps,
+// lane-interleaved (sh_unpack.hip).
+constexpr uint32_t kStepI8F32 = 4;
+constexpr uint32_t kStepB16 = 4;
 constexpr uint32_t kChunkF32 = SH_CHUNK_F32;   // fp32 elements per thread per chunk (cast)
-constexpr uint32_t kChunkB16 = 16;             // bf16 elements per thread per chunk (widen)
+constexpr uint32_t kChunkB16 = 16;             // bf16 elements per thread (widen), in steps of kStepB16
 // Byte kinds, per thread per chunk (measured on a 4 GiB region: copy 16 B
 // 6.57 TB/s vs 32 B 5.90 and 64 B 5.30; zero fill 32 B 6.29 TB/s vs 16 B 5.08
 // and 64 B 5.76).
