@@ -59,17 +59,22 @@ uint32_t dst_elem_bytes(uint32_t kind) {
 //   8.8%; on the config-2 slab, 4 KiB against 64-byte alignment raised the dequant from 6.44-6.48
 //   to 6.55-6.57 TB/s and the cast from 6.19-6.21 to 6.26-6.28.
 // The lead is below one tile for every kind (at most 4095 destination bytes), so a region gains
-// at most one tile. It keeps chunks in their place relative to the region (a multiple of the
-// chunk), so a region whose start allows no such lead gets none. 64 bytes of destination are a
-// whole number of chunks for every kind, so a region that could be put on a 64-byte line can be
-// put on a kDstAlign boundary.
+// at most one tile. A lead that is a whole number of chunks keeps every chunk whole and, where rows
+// are whole chunks, inside one row, so any region gets one. Another lead cuts the region's first
+// chunk (written element by element) and makes int8 chunks cross rows, so only a region of
+// kMinRaggedLead elements or more gets one: 16 tiles of dequant, of which it adds at most one.
+// Measured: a slab of 40 fp32 tensors of odd sizes (hidden 2575) 487 us without and 460 with such
+// leads, the same of int8 245 and 225, 128 int8 tensors of hidden 2999 1064 and 974 us; a block of
+// 128K elements in all is bound by its launch either way. A region whose start is no whole number
+// of elements into the boundary gets none.
 constexpr uint64_t kDstAlign = 4096;
-uint32_t lead_of(uint32_t kind, uint64_t dst_off) {
+constexpr uint64_t kMinRaggedLead = 1ull << 17;
+uint32_t lead_of(uint32_t kind, uint64_t dst_off, uint64_t numel, bool ragged) {
   const uint64_t ob = dst_elem_bytes(kind);
   const uint64_t mis = dst_off % kDstAlign;
   if (mis == 0 || mis % ob != 0) return 0;
   const uint64_t lead = mis / ob;
-  return lead % chunk_of(kind) == 0 ? (uint32_t)lead : 0u;
+  return lead % chunk_of(kind) == 0 || (ragged && numel >= kMinRaggedLead) ? (uint32_t)lead : 0u;
 }
 
 }  // namespace
@@ -84,10 +89,9 @@ struct sh_plan {
 
 namespace {
 
-// Validates the caller's descriptors and produces the launch table (oversize
-// regions split, tiles assigned) and its summary. Host only: no device calls.
-int build_table(const sh_unpack_desc* descs, uint32_t n, std::vector<sh_unpack_desc>& table,
-                sh_plan_info& info, const char* who) {
+// build_table with or without leads that are no whole number of chunks.
+int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool ragged_leads, std::vector<sh_unpack_desc>& table,
+                   sh_plan_info& info, const char* who) {
   if (n > 0 && descs == nullptr) return sh::fail(SH_ERR_INVALID, "%s: descs is NULL", who);
   table.clear();
   table.reserve(n);
@@ -98,7 +102,7 @@ int build_table(const sh_unpack_desc* descs, uint32_t n, std::vector<sh_unpack_d
   auto push = [&](sh_unpack_desc d) -> int {
     const uint64_t numel = (uint64_t)d.rows * d.cols;
     d.div_magic = sh::udiv_magic(d.cols);
-    d.lead = lead_of(d.kind, d.dst_off);
+    d.lead = lead_of(d.kind, d.dst_off, numel, ragged_leads);
     const uint64_t per_tile = tile_of(d.kind);
     const uint64_t nt = (numel + d.lead + per_tile - 1) / per_tile;
     // one workgroup of kThreads work-items per tile, in a 1-D grid: the launch must stay
@@ -172,13 +176,25 @@ int build_table(const sh_unpack_desc* descs, uint32_t n, std::vector<sh_unpack_d
   return SH_OK;
 }
 
+// Validates the caller's descriptors and produces the launch table (oversize
+// regions split, tiles assigned) and its summary. Host only: no device calls.
+// Leads that are no whole number of chunks may add a tile per region; where that
+// takes the table past max_tiles, it is built without them.
+int build_table(const sh_unpack_desc* descs, uint32_t n, uint32_t max_tiles, std::vector<sh_unpack_desc>& table,
+                sh_plan_info& info, const char* who) {
+  const int st = build_table_as(descs, n, true, table, info, who);
+  if (st == SH_OK && info.n_tiles <= max_tiles) return SH_OK;
+  sh::clear_error();
+  return build_table_as(descs, n, false, table, info, who);
+}
+
 }  // namespace
 
 extern "C" int sh_plan_describe(const sh_unpack_desc* descs, uint32_t n, sh_plan_info* info) {
   sh::clear_error();
   if (info == nullptr) return sh::fail(SH_ERR_INVALID, "sh_plan_describe: info is NULL");
   std::vector<sh_unpack_desc> table;
-  return build_table(descs, n, table, *info, "sh_plan_describe");
+  return build_table(descs, n, kMaxTiles, table, *info, "sh_plan_describe");
 }
 
 extern "C" int sh_plan_create(const sh_unpack_desc* descs, uint32_t n, sh_plan** out) {
@@ -187,7 +203,7 @@ extern "C" int sh_plan_create(const sh_unpack_desc* descs, uint32_t n, sh_plan**
   *out = nullptr;
   std::vector<sh_unpack_desc> table;
   sh_plan_info info{};
-  if (int st = build_table(descs, n, table, info, "sh_plan_create")) return st;
+  if (int st = build_table(descs, n, kMaxTiles, table, info, "sh_plan_create")) return st;
   const uint64_t tiles = info.n_tiles;
 
   sh_plan* plan = new (std::nothrow) sh_plan();
@@ -352,7 +368,7 @@ extern "C" int sh_unpack_noalloc(const sh_unpack_desc* descs, uint32_t n, const 
   }
   std::vector<sh_unpack_desc>& table = *g_noalloc_table;
   sh_plan_info in{};
-  if (int st = build_table(descs, n, table, in, who)) return st;
+  if (int st = build_table(descs, n, SH_UNPACK_NOALLOC_MAX_TILES, table, in, who)) return st;
   if (table.size() > SH_UNPACK_NOALLOC_MAX_DESCS)
     return sh::fail(SH_ERR_INVALID, "%s: the plan needs %zu descriptors after splitting; at most %u fit the scratch",
                     who, table.size(), (unsigned)SH_UNPACK_NOALLOC_MAX_DESCS);

@@ -4,7 +4,10 @@ bit for bit, with canary bytes on both sides.
 The sizes sit where the kernels' paths meet: rows one element shorter, equal to and longer than a
 chunk (8 int8 to bf16, 4 to fp32), chunks that end exactly at a row's end, a source that ends with
 the last row's last element, and regions of one tile and one element more. Scales that make NaNs and
-infinities lie beside ordinary ones, in chunks of one row and of two."""
+infinities lie beside ordinary ones, in chunks of one row and of two.
+
+Regions just below and above 131072 elements: from there on a region's tiles start on a destination
+boundary whatever the region's start, and its first chunk is cut."""
 from __future__ import annotations
 
 import numpy as np
@@ -13,8 +16,12 @@ import torch
 
 from oracle import squareq as oq
 from stagehand_amd.unpack import (
+    KIND_BF16_F32,
+    KIND_COPY_BYTES,
+    KIND_F32_BF16,
     KIND_I8_ROWSCALE_BF16,
     KIND_I8_ROWSCALE_F32,
+    KIND_ZERO_BYTES,
     UnpackPlan,
     make_descs,
 )
@@ -63,3 +70,35 @@ def test_rows_of_any_length_stride_and_start(rows, cols, pad, out, start, zp):
         np.testing.assert_array_equal(np.where(np.isnan(body), 0, body).view(np.uint32),
                                       np.where(np.isnan(want), 0, want).view(np.uint32))
     assert (got[:dst_off] == 0xAB).all() and (got[dst_off + rows * cols * width:] == 0xAB).all()
+
+
+@pytest.mark.parametrize("numel", [1, 5, 8193, (1 << 17) - 1, 1 << 17, (1 << 17) + 4099])
+@pytest.mark.parametrize("start", [0, 1, 3, 16, 2047])
+def test_flat_regions_from_any_start(numel, start):
+    """Every flat kind in one plan, each region ``start`` elements past a 4 KiB boundary."""
+    rng = np.random.default_rng(numel + start)
+    f = rng.normal(0, 1, numel).astype(np.float32)
+    bf = oq.cast_f32_bf16(rng.normal(0, 1, numel).astype(np.float32))
+    raw = rng.integers(0, 256, numel, dtype=np.uint8)
+    parts = [f.view(np.uint8), bf.view(np.uint8), raw]
+    src = np.concatenate([np.zeros(3, np.uint8)] + parts)
+    at = np.cumsum([3] + [p.size for p in parts])
+    kinds = [(KIND_F32_BF16, 2), (KIND_BF16_F32, 4), (KIND_COPY_BYTES, 1), (KIND_ZERO_BYTES, 1)]
+    descs, spans, pos = [], [], 0
+    for i, (kind, width) in enumerate(kinds):
+        pos = -(-pos // 4096) * 4096 + width * start
+        descs.append((kind, int(at[i]) if i < 3 else 0, pos, 1, numel, 0, 0))
+        spans.append((pos, pos + width * numel))
+        pos += width * numel
+    dst = torch.full((pos + 4096,), 0xAB, dtype=torch.uint8, device="cuda")
+    UnpackPlan(make_descs(descs)).run(_dev(src), dst)
+    got = dst.cpu().numpy()
+    body = [got[a:b] for a, b in spans]
+    np.testing.assert_array_equal(body[0].view(np.uint16), oq.cast_f32_bf16(f))
+    np.testing.assert_array_equal(body[1].view(np.float32), oq.bf16_bits_to_f32(bf))
+    np.testing.assert_array_equal(body[2], raw)
+    assert not body[3].any()
+    outside = np.ones(got.size, bool)
+    for a, b in spans:
+        outside[a:b] = False
+    assert (got[outside] == 0xAB).all()
