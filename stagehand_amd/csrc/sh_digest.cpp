@@ -27,10 +27,13 @@
 // 32-bit mixers, not 64-bit ones: the kernel is bound by its vector ALU, and a 64-bit multiply
 // is three multiply instructions (v_mad_u64_u32 and two v_mul_lo_u32) against one. Measured on
 // MI355X over a 740 MiB block: 64-bit SplitMix64/Murmur3 mixers 0.147-0.151 ms (5.1-5.3 TB/s);
-// these 0.139-0.142 ms (5.45-5.58 TB/s), and with non-temporal loads 0.126-0.127 ms (6.1 TB/s).
+// these 0.139-0.142 ms (5.45-5.58 TB/s), with non-temporal loads 0.126-0.127 ms (6.1 TB/s), and with
+// the workgroups of threads_for 0.118 ms (6.6 TB/s; the same loop without its mixing 0.114).
+// A multiply from 16-bit products (v_dot2_u32_u16, v_mad_u32_u16) is slower than v_mul_lo_u32.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 
@@ -45,6 +48,28 @@ static_assert(kMaxChunks == 0xFFFFFFFFull / kDigestThreads, "one workgroup per c
 
 uint64_t chunks_of(uint64_t bytes, uint32_t chunk_bytes) {
   return bytes / chunk_bytes + (bytes % chunk_bytes != 0 ? 1 : 0);
+}
+
+// Work-items of each chunk's workgroup, by the number of chunks (MI355X: 256 compute units, each with
+// room for 28 wavefronts of these kernels' registers).
+// - Fewer chunks than compute units: each chunk has a compute unit to itself and its mixing takes all
+//   of its vector ALU, so the more wavefronts hide each other's latency the better. 49 chunks of 256
+//   KiB (digest and comparison) 21.6 us with 1024, 23.6 with 512, 34.3 with 256 work-items; 16 chunks
+//   of 1 MiB 67, 76 and 120.
+// - Up to one and a half chunks per compute unit: 256 chunks of 256 KiB 29.6, 26.9 and 37.7 us; 384
+//   chunks 46.4, 43.3 and 44.1 us.
+// - More: 256 work-items, the most workgroups in flight, are the fastest (512 chunks 53.6, 51.4 and
+//   46.6 us), but a compute unit then holds 7 chunks, and with more than 7 * 256 of them the last round
+//   leaves many idle. 768 work-items hold 2 and lose less: 2048 chunks of 256 KiB 166 against 177 us,
+//   2960 chunks 236 against 241. Chunks under 256 KiB are too few 768-wide steps to divide evenly:
+//   2048 chunks of 64 KiB 53.5 us with 768, 49.4 with 256.
+// Never so many that a work-item of a whole chunk has fewer than four 16-byte words.
+uint32_t threads_for(uint64_t n, uint64_t bytes, uint32_t chunk_bytes) {
+  const uint64_t words = std::min<uint64_t>(bytes, chunk_bytes) / 16;
+  if (n < 256 && words >= 4 * kDigestMaxThreads) return kDigestMaxThreads;
+  if (n <= 384 && words >= 4 * 512) return 512;
+  if (n > 7 * 256 && n <= 0xFFFFFFFFull / 768 && chunk_bytes >= (1u << 18)) return 768;
+  return kDigestThreads;
 }
 
 int check_args(const void* buf, uint64_t bytes, uint32_t chunk_bytes, const void* digests, const char* who) {
@@ -69,8 +94,9 @@ int launch_block_changed(const void* buf, uint64_t bytes, uint32_t chunk_bytes, 
   if (bytes == 0) return SH_OK;
   const uint8_t* b = (const uint8_t*)buf;
   uint64_t chunk = chunk_bytes;
+  const uint64_t n = chunks_of(bytes, chunk_bytes);
   void* args[] = {(void*)&b, (void*)&bytes, (void*)&chunk, (void*)&digests, (void*)&changed};
-  return launch_kernel(kKernDigestCompare, (uint32_t)chunks_of(bytes, chunk_bytes), kDigestThreads, stream, args,
+  return launch_kernel(kKernDigestCompare, (uint32_t)n, threads_for(n, bytes, chunk_bytes), stream, args,
                        "sh_block_changed");
 }
 
@@ -80,9 +106,9 @@ int launch_block_digest(const void* buf, uint64_t bytes, uint32_t chunk_bytes, u
   if (bytes == 0) return SH_OK;
   const uint8_t* b = (const uint8_t*)buf;
   uint64_t chunk = chunk_bytes;
+  const uint64_t n = chunks_of(bytes, chunk_bytes);
   void* args[] = {(void*)&b, (void*)&bytes, (void*)&chunk, (void*)&digests};
-  return launch_kernel(kKernDigest, (uint32_t)chunks_of(bytes, chunk_bytes), kDigestThreads, stream, args,
-                       "sh_block_digest");
+  return launch_kernel(kKernDigest, (uint32_t)n, threads_for(n, bytes, chunk_bytes), stream, args, "sh_block_digest");
 }
 
 }  // namespace sh

@@ -10,7 +10,8 @@
 namespace {
 
 constexpr uint32_t kKey = 0x9E3779B9u;  // word j's key is j * kKey mod 2^32
-constexpr uint32_t kDigestThreads = 256;
+constexpr uint32_t kDigestThreads = 256;  // work-items per chunk of a long launch
+constexpr uint32_t kDigestMaxThreads = 1024;
 
 // MurmurHash3's 32-bit finalizer (Austin Appleby, public domain).
 __host__ __device__ inline uint32_t mix_f(uint32_t x) {
