@@ -80,6 +80,8 @@ enum KernelId : int {
   kKernCastBf16,
   kKernMixed,
   kKernMixedZp,
+  kKernUnpackArgs,
+  kKernUnpackArgsZp,
   kKernPutDescs,
   kKernFillTileMap,
   kKernDigest,

@@ -95,4 +95,11 @@ struct DescChunk {
   uint32_t count;
 };
 
+// A whole launch table of at most kDescChunk descriptors as kernel arguments; tile_begin repeats the
+// descriptors' field, 0xFFFFFFFF (above every tile) past the last one.
+struct DescArgs {
+  uint32_t tile_begin[kDescChunk];
+  sh_unpack_desc d[kDescChunk];
+};
+
 }  // namespace

@@ -174,12 +174,13 @@ def unpack_noalloc(
     stream: torch.cuda.Stream | int | None = None,
 ) -> None:
     """``dst`` ← unpack(``src``) for the descriptor table ``descs``, allocating no device memory
-    (``sh_unpack_noalloc``: the launch table lives in the library's static per-GPU scratch).
+    (``sh_unpack_noalloc``: a short table travels in the launch's arguments, a longer one lives in the
+    library's static per-GPU scratch).
 
     The results equal an :class:`UnpackPlan` of the same table run with ``sh_unpack``. Calls on one
-    GPU share the scratch; each call's kernels wait on the device for the previous call's, from
-    any stream or thread. A call recorded into a graph is not ordered that way: replays of such a
-    graph must not overlap other calls on that GPU."""
+    GPU with tables of more than 32 descriptors or 32768 tiles share the scratch; each one's kernels
+    wait on the device for the previous one's, from any stream or thread. Such a call recorded into
+    a graph is not ordered that way: replays of the graph must not overlap others on that GPU."""
     table = np.ascontiguousarray(descs, dtype=DESC_DTYPE)
     sp, sb = _device_ptr(src, "src")
     dp, db = _device_ptr(dst, "dst")

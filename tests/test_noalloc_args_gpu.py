@@ -1,0 +1,115 @@
+"""``sh_unpack_noalloc`` around the limits of a table that travels in the launch's arguments (32
+descriptors, 32768 tiles): the same bytes as the plan-based entry point on both sides of them, on two
+streams at once, and at every replay of a captured call."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from stagehand_amd.unpack import (
+    KIND_BF16_F32,
+    KIND_COPY_BYTES,
+    KIND_F32_BF16,
+    KIND_I8_ROWSCALE_BF16,
+    KIND_I8_ROWSCALE_F32,
+    KIND_ZERO_BYTES,
+    UnpackPlan,
+    make_descs,
+    unpack_noalloc,
+)
+
+pytestmark = pytest.mark.gpu
+
+KINDS = [(KIND_I8_ROWSCALE_BF16, 1, 2), (KIND_F32_BF16, 4, 2), (KIND_I8_ROWSCALE_F32, 1, 4), (KIND_BF16_F32, 2, 4),
+         (KIND_COPY_BYTES, 1, 1), (KIND_ZERO_BYTES, 0, 1)]
+
+
+def _table(n: int, kinds=KINDS):
+    """n regions of changing kind and size (one element to several tiles); (descs, source bytes,
+    destination bytes, scales)."""
+    rows, src, dst, scale = [], 3, 0, 0
+    for i in range(n):
+        kind, ib, ob = kinds[i % len(kinds)]
+        r, c = (5 + i, 77 + 613 * (i % 7)) if kind in (KIND_I8_ROWSCALE_BF16, KIND_I8_ROWSCALE_F32) else (1, 1 + 3001 * i)
+        dst = -(-dst // ob) * ob
+        rows.append((kind, src if ib else 0, dst, r, c, 0, scale))
+        src += r * c * ib
+        dst += r * c * ob
+        scale += r
+    return make_descs(rows), src, dst, scale
+
+
+def _inputs(src_bytes: int, n_scale: int, seed: int):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    src = torch.randint(0, 256, (src_bytes + 16,), dtype=torch.uint8, device="cuda", generator=g)
+    return src, torch.rand(max(n_scale, 1), device="cuda", generator=g), torch.randn(max(n_scale, 1), device="cuda", generator=g)
+
+
+def _want(descs, src, dst_bytes, scales, zps):
+    want = torch.full((dst_bytes + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    plan = UnpackPlan(descs)
+    plan.run(src, want, scales, zps)
+    plan.close()
+    return want
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 31, 32, 33])
+@pytest.mark.parametrize("zp", [False, True])
+def test_tables_on_both_sides_of_the_argument_limit(n, zp):
+    descs, sb, db, ns = _table(n)
+    src, scales, zps = _inputs(sb, ns, n)
+    want = _want(descs, src, db, scales, zps if zp else None)
+    got = torch.full_like(want, 0xA5)
+    unpack_noalloc(descs, src, got, scales, zps if zp else None)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tiles", [32768, 32769])
+def test_tile_limit_of_the_arguments(tiles):
+    n = 8192 * tiles
+    src = torch.arange(n // 8, device="cuda").view(torch.uint8)
+    got = torch.zeros_like(src)
+    unpack_noalloc(make_descs([(KIND_COPY_BYTES, 0, 0, 1, n, 0, 0)]), src, got)
+    assert torch.equal(got, src)
+
+
+def test_short_and_long_tables_on_two_streams():
+    cases = []
+    for n in (32, 40, 3, 64):
+        descs, sb, db, ns = _table(n)
+        src, scales, _z = _inputs(sb, ns, n)
+        cases.append((descs, src, scales, _want(descs, src, db, scales, None)))
+    outs = [[torch.full_like(c[3], 0xA5) for c in cases] for _ in range(2)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for i in range(len(cases)):
+        for j, stream in enumerate(streams):
+            descs, src, scales, _w = cases[(i + j) % len(cases)]
+            unpack_noalloc(descs, src, outs[j][(i + j) % len(cases)], scales, stream=stream)
+    torch.cuda.synchronize()
+    for out in outs:
+        for got, case in zip(out, cases):
+            assert torch.equal(got, case[3])
+
+
+def test_captured_call_at_every_replay():
+    descs, sb, db, ns = _table(12)
+    src, scales, _z = _inputs(sb, ns, 1)
+    got = torch.full((db + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    unpack_noalloc(descs, src, got, scales)  # kernels loaded before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        unpack_noalloc(descs, src, got, scales)
+    other, osb, odb, ons = _table(20)
+    osrc, oscales, _z = _inputs(osb, ons, 2)
+    for seed in range(3, 6):
+        src.copy_(_inputs(sb, ns, seed)[0])
+        got.fill_(0xA5)
+        want = _want(descs, src, db, scales, None)
+        graph.replay()
+        eager = torch.empty(odb, dtype=torch.uint8, device="cuda")
+        unpack_noalloc(other, osrc, eager, oscales)  # an eager call between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
