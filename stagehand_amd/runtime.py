@@ -32,6 +32,7 @@ from stagehand_amd.residency import ResidencyMap
 from stagehand_amd.scheduler import StagehandScheduler, StaticLookaheadPolicy
 from stagehand_amd.telemetry import StagehandTelemetry
 from stagehand_amd.transfer import AsyncTransferEngine
+from stagehand_amd.unpack import current_stream_handle
 
 __all__ = ["StagehandRuntime", "layer", "wrap", "Runtime"]
 
@@ -226,7 +227,7 @@ class StagehandRuntime:
         if idx is None:
             return False
         handle = self._vmm.models[self._vmm_model_id]
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = current_stream_handle()
         tensor, ok = handle.get_block_tensor(idx, stream)
         # the next block's fill runs while this one computes; further blocks of the prefetch
         # window only while they fit under the ceiling without evicting anything

@@ -41,6 +41,7 @@ from stagehand_amd.fileio import FileCache, FileRange
 from stagehand_amd.residency import BlockState
 from stagehand_amd.staging import PlanCache, SourceBuilder, squareq_weight_tensors
 from stagehand_amd.transfer import NativeEvent
+from stagehand_amd.unpack import current_stream_handle
 
 if TYPE_CHECKING:
     from stagehand_amd.config import StagehandConfig
@@ -639,7 +640,7 @@ class StagehandScheduler:
     def _mark_block_done(self) -> None:
         if self._has_cuda and self._run_ahead_limit() > 0:
             ev = NativeEvent()
-            ev.record(torch.cuda.current_stream().cuda_stream)
+            ev.record(current_stream_handle())
             self._done_marks.append(ev)
 
     def before_block(self, block_id: str) -> None:
@@ -1101,7 +1102,7 @@ class StagehandScheduler:
             if d2h_fence is not None and any(p.grad is not None and p.grad.device.type == "cpu"
                                              for p in module.parameters()):
                 # saved-back gradients move to the device on the current stream, after their save-back
-                d2h_fence.wait_on(torch.cuda.current_stream().cuda_stream)
+                d2h_fence.wait_on(current_stream_handle())
             if getattr(self._config, "frozen_host_copies", False):
                 params = dict(module.named_parameters())
                 keep = {}

@@ -38,6 +38,7 @@ import torch
 from stagehand_amd import _native
 from stagehand_amd._native import COPY_ITEM_DTYPE, FILE_RANGE_DTYPE, LOAD_REQUEST_DTYPE
 from stagehand_amd.errors import TransferError
+from stagehand_amd.unpack import current_stream_handle as _current_stream_handle
 
 if TYPE_CHECKING:
     from stagehand_amd.pool import PinnedPool, PinnedSlab
@@ -250,10 +251,6 @@ class BlockSource:
     # change between loads (module parameters); None key = not cacheable
     key: bytes | None = None
     mutable: frozenset = frozenset()
-
-
-def _current_stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 class AsyncTransferEngine:

@@ -29,6 +29,7 @@ import torch
 from torch import nn
 
 from stagehand_amd import _native
+from stagehand_amd.unpack import current_stream_handle
 
 __all__ = ["TransferEngine", "TurboConductor", "is_available"]
 
@@ -49,7 +50,7 @@ def is_available() -> bool:
 
 def _stream_handle(stream) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else 0
+        return current_stream_handle() if torch.cuda.is_available() else 0
     return stream if isinstance(stream, int) else stream.cuda_stream
 
 

@@ -63,16 +63,24 @@ def make_descs(rows: Iterable[Sequence[int]]) -> np.ndarray:
 def _device_ptr(t: torch.Tensor | None, what: str) -> tuple[int, int]:
     if t is None:
         return 0, 0
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{what} must be a device tensor, got {t.device}")
     if not t.is_contiguous():
         raise ValueError(f"{what} must be contiguous")
-    return t.data_ptr(), t.numel() * t.element_size()
+    return t.data_ptr(), t.nbytes
+
+
+def current_stream_handle() -> int:
+    """``torch.cuda.current_stream().cuda_stream``, without building the stream object: that takes 2.5
+    us, a third of a small unpack call (7.8 us on the host, 4.8 with this); the two lookups 0.15."""
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _stream_handle(stream: torch.cuda.Stream | int | None) -> int:
     if stream is None:
-        return torch.cuda.current_stream().cuda_stream
+        return current_stream_handle()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
