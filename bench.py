@@ -713,17 +713,18 @@ def _dit_run(kind: str, args, src: Path, layers, pinned: bool, reader: str = "mm
 
 
 def trace_marker(args) -> None:
-    """With ``--trace-markers``: one allocation-free unpack of 16 zero bytes, whose
-    ``sh_put_descs_kernel`` launch runs nowhere else in a streamed step. Placed before and after the
-    timed steps, the two launches bound them in a rocprofv3 kernel trace (``--trace-summary``)."""
+    """With ``--trace-markers``: one allocation-free unpack of a table too long for one launch's
+    arguments (33 regions of 16 zero bytes), whose ``sh_put_descs_kernel`` launches run nowhere else
+    in a streamed step. Placed before and after the timed steps, the first and the last of them bound
+    the steps in a rocprofv3 kernel trace (``--trace-summary``)."""
     if not getattr(args, "trace_markers", False):
         return
     import torch
 
     from stagehand_amd.unpack import KIND_ZERO_BYTES, make_descs, unpack_noalloc
 
-    buf = torch.empty(16, dtype=torch.uint8, device="cuda")
-    unpack_noalloc(make_descs([(KIND_ZERO_BYTES, 0, 0, 1, 16, 0, 0)]), None, buf)
+    buf = torch.empty(33 * 16, dtype=torch.uint8, device="cuda")
+    unpack_noalloc(make_descs([(KIND_ZERO_BYTES, 0, 16 * i, 1, 16, 0, 0) for i in range(33)]), None, buf)
     torch.cuda.synchronize()
 
 
