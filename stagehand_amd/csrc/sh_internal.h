@@ -78,6 +78,7 @@ enum KernelId : int {
   kKernDequantBf16 = 0,
   kKernDequantBf16Zp,
   kKernCastBf16,
+  kKernCastBf16Short,
   kKernMixed,
   kKernMixedZp,
   kKernUnpackArgs,

@@ -371,6 +371,10 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
 
 // ── fp32 → bf16 cast ──────────────────────────────────────────────────────
 
+// SHORT: a launch whose output the memory-side cache can hold a good part of; it stores past the L2
+// (nt) too. Measured (MI355X; plain against nt stores): 25 MB 5.2 and 4.9 us, 57 MB 12.5 and 10.5, 126
+// MB 24.5 and 22.5, 354 MB 61.6 and 59.4, 510 MB the same, 1 GB 165.0 and 165.8, 13 GB 2099 and 2158.
+template <bool SHORT>
 __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t local,
                                               const uint8_t* __restrict__ src,
                                               uint8_t* __restrict__ dst) {
@@ -394,7 +398,10 @@ __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t 
 #pragma unroll
       for (uint32_t w = 0; w < C / 2; ++w)
         ow.w[w] = pack_hi(rne_hi_nan(__uint_as_float(v[k].w[2 * w])), rne_hi_nan(__uint_as_float(v[k].w[2 * w + 1])));
-      stw<2 * C>(o + (size_t)e * 2, ow);
+      if constexpr (SHORT)
+        stw_nt<2 * C>(o + (size_t)e * 2, ow);
+      else
+        stw<2 * C>(o + (size_t)e * 2, ow);
     } else {
 #pragma unroll 1
       for (uint32_t j = e; j != e + C; ++j) {  // cut by the region's start or end
@@ -508,7 +515,7 @@ __device__ __forceinline__ sh_unpack_desc load_desc(const sh_unpack_desc* __rest
   return d;
 }
 
-template <uint32_t MASK, bool HAS_ZP>
+template <uint32_t MASK, bool HAS_ZP, bool SHORT>
 __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t tile,
                                             const uint8_t* __restrict__ src,
                                             const float* __restrict__ scales,
@@ -522,7 +529,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
     return;
   }
   if constexpr (MASK == kMaskCastBf16) {
-    tile_f32_bf16(d, local, src, dst);
+    tile_f32_bf16<SHORT>(d, local, src, dst);
     return;
   }
   switch (d.kind) {
@@ -535,7 +542,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
         tile_i8<false, HAS_ZP, false>(d, local, src, scales, zps, dst);
       break;
     case SH_KIND_F32_BF16:
-      if constexpr ((MASK & bit(SH_KIND_F32_BF16)) != 0) tile_f32_bf16(d, local, src, dst);
+      if constexpr ((MASK & bit(SH_KIND_F32_BF16)) != 0) tile_f32_bf16<SHORT>(d, local, src, dst);
       break;
     case SH_KIND_BF16_F32:
       if constexpr ((MASK & bit(SH_KIND_BF16_F32)) != 0) tile_bf16_f32(d, local, src, dst);
@@ -551,7 +558,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
   }
 }
 
-template <uint32_t MASK, bool HAS_ZP>
+template <uint32_t MASK, bool HAS_ZP, bool SHORT = false>
 __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ descs,
                                             const uint32_t* __restrict__ tile_map,
                                             const uint8_t* __restrict__ src,
@@ -559,7 +566,7 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
                                             const float* __restrict__ zps,
                                             uint8_t* __restrict__ dst) {
   const uint32_t tile = blockIdx.x;
-  unpack_tile<MASK, HAS_ZP>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
+  unpack_tile<MASK, HAS_ZP, SHORT>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
 }
 
 // The launch table in the kernel's arguments: the descriptor of a tile is the last one whose
@@ -576,7 +583,7 @@ __device__ __forceinline__ void unpack_args_body(const DescArgs& a, const uint8_
 #pragma unroll
   for (uint32_t step = kDescChunk / 2; step > 0; step /= 2)
     if (a.tile_begin[i + step] <= tile) i += step;
-  unpack_tile<kMaskAll, HAS_ZP>(load_desc(a.d + i), tile, src, scales, zps, dst);
+  unpack_tile<kMaskAll, HAS_ZP, true>(load_desc(a.d + i), tile, src, scales, zps, dst);
 }
 
 }  // namespace
@@ -594,6 +601,9 @@ extern "C" __global__ __launch_bounds__(kThreads) void sh_dequant_i8_bf16_zp_ker
 }
 extern "C" __global__ __launch_bounds__(kThreads) void sh_cast_f32_bf16_kernel(SH_KERNEL_ARGS) {
   unpack_body<kMaskCastBf16, false>(descs, tile_map, src, scales, zps, dst);
+}
+extern "C" __global__ __launch_bounds__(kThreads) void sh_cast_f32_bf16_short_kernel(SH_KERNEL_ARGS) {
+  unpack_body<kMaskCastBf16, false, true>(descs, tile_map, src, scales, zps, dst);
 }
 extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_kernel(SH_KERNEL_ARGS) {
   unpack_body<kMaskAll, false>(descs, tile_map, src, scales, zps, dst);

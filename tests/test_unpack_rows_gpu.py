@@ -102,3 +102,16 @@ def test_flat_regions_from_any_start(numel, start):
     for a, b in spans:
         outside[a:b] = False
     assert (got[outside] == 0xAB).all()
+
+
+@pytest.mark.parametrize("numel", [2048 * 32768, 2048 * 32768 + 1])
+def test_cast_on_both_sides_of_the_kernel_choice(numel):
+    """A cast-only plan takes another kernel above 32768 tiles of 2048 elements; torch's device cast
+    rounds the same way (no NaN here)."""
+    g = torch.Generator(device="cuda").manual_seed(numel)
+    src = torch.randn(numel, device="cuda", generator=g)
+    dst = torch.empty(numel, dtype=torch.bfloat16, device="cuda")
+    plan = UnpackPlan(make_descs([(KIND_F32_BF16, 0, 0, 1, numel, 0, 0)]))
+    assert plan.info["n_tiles"] == -(-numel // 2048)
+    plan.run(src, dst)
+    assert torch.equal(dst, src.to(torch.bfloat16))
