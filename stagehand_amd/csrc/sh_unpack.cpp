@@ -61,12 +61,14 @@ uint32_t dst_elem_bytes(uint32_t kind) {
 // The lead is below one tile for every kind (at most 4095 destination bytes), so a region gains
 // at most one tile. A lead that is a whole number of chunks keeps every chunk whole and, where rows
 // are whole chunks, inside one row, so any region gets one. Another lead cuts the region's first
-// chunk (written element by element) and makes int8 chunks cross rows, so only a region of
-// kMinRaggedLead elements or more gets one: 16 tiles of dequant, of which it adds at most one.
-// Measured: a slab of 40 fp32 tensors of odd sizes (hidden 2575) 487 us without and 460 with such
-// leads, the same of int8 245 and 225, 128 int8 tensors of hidden 2999 1064 and 974 us; a block of
-// 128K elements in all is bound by its launch either way. A region whose start is no whole number
-// of elements into the boundary gets none.
+// chunk (written element by element) and makes int8 chunks cross rows, so only a dequant, cast
+// or widen of kMinRaggedLead elements or more gets one: 16 tiles of dequant, of which it adds at
+// most one. Measured: a slab of 40 fp32 tensors of odd sizes (hidden 2575) 487 us without and 460 with such
+// leads, the same of int8 245 and 225, 128 int8 tensors of hidden 2999 1064 and 974 us, a widen of 64
+// M elements 62.2 and 58.1; a block of 128K elements in all is bound by its launch either way. A byte
+// copy loses by it, as its loads go off their 16 bytes when its stores come onto them (256 MiB 88
+// us without and 95 with), and zero fill gains nothing. A region whose start is no whole number of elements into the
+// boundary gets none.
 constexpr uint64_t kDstAlign = 4096;
 constexpr uint64_t kMinRaggedLead = 1ull << 17;
 uint32_t lead_of(uint32_t kind, uint64_t dst_off, uint64_t numel, bool ragged) {
@@ -74,7 +76,8 @@ uint32_t lead_of(uint32_t kind, uint64_t dst_off, uint64_t numel, bool ragged) {
   const uint64_t mis = dst_off % kDstAlign;
   if (mis == 0 || mis % ob != 0) return 0;
   const uint64_t lead = mis / ob;
-  return lead % chunk_of(kind) == 0 || (ragged && numel >= kMinRaggedLead) ? (uint32_t)lead : 0u;
+  const bool gains = is_i8(kind) || kind == SH_KIND_F32_BF16 || kind == SH_KIND_BF16_F32;
+  return lead % chunk_of(kind) == 0 || (ragged && gains && numel >= kMinRaggedLead) ? (uint32_t)lead : 0u;
 }
 
 }  // namespace

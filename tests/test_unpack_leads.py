@@ -1,6 +1,7 @@
 """Where a plan's tiles start in a region whose destination is no whole number of chunks past a 4 KiB
-boundary (CPU only: ``sh_plan_describe``). From 131072 elements on, the lead before element 0 reaches
-back to the boundary all the same; below, such a region gets none."""
+boundary (CPU only: ``sh_plan_describe``). From 131072 elements on, the lead of a dequant, cast or widen
+before element 0 reaches back to the boundary all the same; shorter regions and the other kinds (a
+byte copy is slower so) get none."""
 from __future__ import annotations
 
 import numpy as np
@@ -21,7 +22,8 @@ from stagehand_amd.unpack import (
 MIN_LEAD = 1 << 17
 # kind: (elements per tile, bytes of an output element)
 KINDS = {KIND_I8_ROWSCALE_BF16: (8192, 2), KIND_I8_ROWSCALE_F32: (8192, 4), KIND_F32_BF16: (2048, 2),
-         KIND_BF16_F32: (8192, 4), KIND_COPY_BYTES: (8192, 1), KIND_ZERO_BYTES: (16384, 1)}
+         KIND_BF16_F32: (8192, 4)}
+NO_LEAD = {KIND_COPY_BYTES: (8192, 1), KIND_ZERO_BYTES: (16384, 1)}
 
 
 def tiles(kind: int, dst_off: int, cols: int, rows: int = 1) -> int:
@@ -37,10 +39,17 @@ def test_a_long_region_gets_a_lead_of_any_length(kind, lead):
     per_tile, width = KINDS[kind]
     for numel in (MIN_LEAD, MIN_LEAD + per_tile - lead, MIN_LEAD + per_tile - lead + 1):
         assert tiles(kind, 4096 + lead * width, numel) == -(-(numel + lead) // per_tile), numel
-        if width > 1:  # starts inside an element's worth of bytes: no lead reaches the boundary
-            assert tiles(kind, 4096 + lead * width + 1, numel) == -(-numel // per_tile)
+        # a start inside an element's worth of bytes: no lead reaches the boundary
+        assert tiles(kind, 4096 + lead * width + 1, numel) == -(-numel // per_tile)
     short = MIN_LEAD - 1 - (MIN_LEAD - 1) % per_tile  # whole tiles, below the line
     assert tiles(kind, 4096 + lead * width, short) == short // per_tile
+
+
+@pytest.mark.parametrize("kind", NO_LEAD)
+def test_the_other_kinds_get_whole_chunk_leads_only(kind):
+    per_tile, width = NO_LEAD[kind]
+    for lead in (1, 3, 5, 1021):
+        assert tiles(kind, 4096 + lead * width, 64 * per_tile) == 64, lead
 
 
 def test_a_lead_never_refuses_a_table_that_fits_without_it():
@@ -49,8 +58,8 @@ def test_a_lead_never_refuses_a_table_that_fits_without_it():
     max_tiles = (2**32 - 1) // 512
     assert tiles(KIND_F32_BF16, 4096 + 2, 2048, rows=max_tiles) == max_tiles
     lib = _native.lib()
-    for rows, message in ((2064384, b"destination"), (2064385, b"tiles")):  # fits: refused for its buffer alone
-        table = make_descs([(KIND_ZERO_BYTES, 0, 4097, rows, 16384, 0, 0)])
+    for rows, message in ((2064384, b"source"), (2064385, b"tiles")):  # fits: refused for its buffers alone
+        table = make_descs([(KIND_F32_BF16, 0, 4098, rows, 2048, 0, 0)])
         assert lib.sh_unpack_noalloc(table.ctypes.data, 1, None, 0, None, None, 0, None, 0,
                                      None) == _native.SH_ERR_INVALID
         assert message in lib.sh_last_error()

@@ -6,8 +6,8 @@ chunk (8 int8 to bf16, 4 to fp32), chunks that end exactly at a row's end, a sou
 the last row's last element, and regions of one tile and one element more. Scales that make NaNs and
 infinities lie beside ordinary ones, in chunks of one row and of two.
 
-Regions just below and above 131072 elements: from there on a region's tiles start on a destination
-boundary whatever the region's start, and its first chunk is cut."""
+Regions just below and above 131072 elements: from there on the tiles of a dequant, cast or widen start
+on a destination boundary whatever the region's start, and its first chunk is cut."""
 from __future__ import annotations
 
 import numpy as np
