@@ -151,10 +151,10 @@ typedef struct sh_unpack_desc {
   /* filled by sh_plan_create: */
   uint64_t div_magic;  /* ceil(2^64 / cols), 0 when cols == 1 */
   uint32_t tile_begin; /* first tile of this descriptor */
-  uint32_t ntiles;     /* tiles covering rows*cols elements */
+  uint32_t ntiles;     /* workgroups covering rows*cols elements */
   uint32_t lead;       /* elements before element 0 in the first tile, so that the tiles' destination
                           spans start on 4 KiB boundaries (0 when the region start allows none) */
-  uint32_t reserved;
+  uint32_t reserved;   /* 1: a workgroup takes two tiles (fp32 outputs of a table near the launch limit) */
 } sh_unpack_desc;     /* 64 bytes, identical layout on host and device */
 
 typedef struct sh_plan sh_plan;

@@ -92,8 +92,9 @@ struct sh_plan {
 
 namespace {
 
-// build_table with or without leads that are no whole number of chunks.
-int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool ragged_leads, std::vector<sh_unpack_desc>& table,
+// build_table in the form that runs fastest, or (fewest) in the one of fewest tiles: no leads that are
+// no whole number of chunks, two tiles to a workgroup of the kinds with fp32 outputs.
+int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool fewest, std::vector<sh_unpack_desc>& table,
                    sh_plan_info& info, const char* who) {
   if (n > 0 && descs == nullptr) return sh::fail(SH_ERR_INVALID, "%s: descs is NULL", who);
   table.clear();
@@ -105,8 +106,9 @@ int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool ragged_leads, s
   auto push = [&](sh_unpack_desc d) -> int {
     const uint64_t numel = (uint64_t)d.rows * d.cols;
     d.div_magic = sh::udiv_magic(d.cols);
-    d.lead = lead_of(d.kind, d.dst_off, numel, ragged_leads);
-    const uint64_t per_tile = tile_of(d.kind);
+    d.lead = lead_of(d.kind, d.dst_off, numel, !fewest);
+    d.reserved = fewest && dst_elem_bytes(d.kind) == 4 ? 1 : 0;
+    const uint64_t per_tile = (uint64_t)tile_of(d.kind) << d.reserved;
     const uint64_t nt = (numel + d.lead + per_tile - 1) / per_tile;
     // one workgroup of kThreads work-items per tile, in a 1-D grid: the launch must stay
     // under 2^32 work-items
@@ -115,7 +117,6 @@ int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool ragged_leads, s
                       who, kMaxTiles, kThreads);
     d.tile_begin = (uint32_t)tiles;
     d.ntiles = (uint32_t)nt;
-    d.reserved = 0;
     tiles += nt;
     const uint32_t ld = d.src_ld ? d.src_ld : d.cols;
     const uint64_t src_span =
@@ -181,14 +182,13 @@ int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool ragged_leads, s
 
 // Validates the caller's descriptors and produces the launch table (oversize
 // regions split, tiles assigned) and its summary. Host only: no device calls.
-// Leads that are no whole number of chunks may add a tile per region; where that
-// takes the table past max_tiles, it is built without them.
+// A table that the fastest form takes past max_tiles is built in the form of fewest tiles.
 int build_table(const sh_unpack_desc* descs, uint32_t n, uint32_t max_tiles, std::vector<sh_unpack_desc>& table,
                 sh_plan_info& info, const char* who) {
-  const int st = build_table_as(descs, n, true, table, info, who);
+  const int st = build_table_as(descs, n, false, table, info, who);
   if (st == SH_OK && info.n_tiles <= max_tiles) return SH_OK;
   sh::clear_error();
-  return build_table_as(descs, n, false, table, info, who);
+  return build_table_as(descs, n, true, table, info, who);
 }
 
 }  // namespace

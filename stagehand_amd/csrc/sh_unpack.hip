@@ -350,10 +350,10 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
                                         const float* __restrict__ zps, uint8_t* __restrict__ dst) {
   // A chunk is one 16-byte store, 8 bf16 or 4 fp32 outputs, so a wavefront's store instruction
   // covers one contiguous 1 KiB span. With 8 fp32 per chunk each lane wrote two 16-byte halves at a
-  // 32-byte stride: a float32 double-stream block (hidden 1536) 84 us, now 62 (6.9 TB/s); plain
-  // instead of non-temporal fp32 stores 76 us.
-  constexpr uint32_t C = OUT_BF16 ? kChunkI8 : kStepI8F32;
-  constexpr uint32_t U = kUnrollI8 * kChunkI8 / C;
+  // 32-byte stride: a float32 double-stream block (hidden 1536) 84 us, now 61 (7.0 TB/s); plain
+  // instead of non-temporal fp32 stores 75 us.
+  constexpr uint32_t C = OUT_BF16 ? kChunkI8 : kStepF32;
+  constexpr uint32_t U = OUT_BF16 ? kUnrollI8 : kPerThreadF32 / C;
   constexpr uint32_t T = kThreads * U * C;
   const uint32_t cols = d.cols;
   const uint32_t numel = d.rows * cols;
@@ -362,11 +362,16 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
   uint8_t* o = dst + d.dst_off;
   const float* sc = scales + d.scale_off;
   const float* zp = HAS_ZP ? zps + d.scale_off : nullptr;
-  const uint32_t e0 = local * T + threadIdx.x * C - d.lead;
-  if (cols >= C)
-    i8_rows<OUT_BF16, HAS_ZP, ALONE, C, U>(d, e0, numel, pad, s, sc, zp, o);
-  else
-    i8_short_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, pad, s, sc, zp, o);
+  // A workgroup takes one tile, or two of an fp32 output where the table is near the launch limit.
+  const uint32_t last = OUT_BF16 ? 0u : d.reserved;
+  uint32_t e0 = (local << last) * T + threadIdx.x * C - d.lead;
+#pragma unroll 1
+  for (uint32_t sub = 0; sub <= last; ++sub, e0 += T) {
+    if (cols >= C)
+      i8_rows<OUT_BF16, HAS_ZP, ALONE, C, U>(d, e0, numel, pad, s, sc, zp, o);
+    else
+      i8_short_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, pad, s, sc, zp, o);
+  }
 }
 
 // ── fp32 → bf16 cast ──────────────────────────────────────────────────────
@@ -417,18 +422,13 @@ __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t 
 
 // ── bf16 → fp32 widen ─────────────────────────────────────────────────────
 
-// A tile is kThreads * kChunkB16 elements, moved kStepB16 at a time (one 16-byte store) with
+// A tile is kThreads * kPerThreadF32 elements, moved kStepF32 at a time (one 16-byte store) with
 // consecutive lanes on consecutive steps, so each store instruction of a wavefront covers one
 // contiguous 1 KiB span.
-__device__ __forceinline__ void tile_bf16_f32(const sh_unpack_desc& d, uint32_t local,
-                                              const uint8_t* __restrict__ src,
-                                              uint8_t* __restrict__ dst) {
-  constexpr uint32_t C = kStepB16;
-  constexpr uint32_t U = kChunkB16 / kStepB16;
-  const uint32_t numel = d.rows * d.cols;
-  const uint8_t* s = src + d.src_off;
-  uint8_t* o = dst + d.dst_off;
-  const uint32_t e0 = local * (kThreads * U * C) + threadIdx.x * C - d.lead;
+__device__ __forceinline__ void bf16_f32_steps(uint32_t e0, uint32_t numel, const uint8_t* __restrict__ s,
+                                               uint8_t* __restrict__ o) {
+  constexpr uint32_t C = kStepF32;
+  constexpr uint32_t U = kPerThreadF32 / C;
   Words<2 * C> v[U];
 #pragma unroll
   for (uint32_t k = 0; k < U; ++k) {
@@ -457,6 +457,17 @@ __device__ __forceinline__ void tile_bf16_f32(const sh_unpack_desc& d, uint32_t 
       }
     }
   }
+}
+
+__device__ __forceinline__ void tile_bf16_f32(const sh_unpack_desc& d, uint32_t local,
+                                              const uint8_t* __restrict__ src,
+                                              uint8_t* __restrict__ dst) {
+  constexpr uint32_t T = kThreads * kPerThreadF32;
+  const uint32_t numel = d.rows * d.cols;
+  uint32_t e0 = (local << d.reserved) * T + threadIdx.x * kStepF32 - d.lead;
+#pragma unroll 1
+  for (uint32_t sub = 0; sub <= d.reserved; ++sub, e0 += T)  // one tile, or two as in tile_i8
+    bf16_f32_steps(e0, numel, src + d.src_off, dst + d.dst_off);
 }
 
 // ── byte copy / zero fill ─────────────────────────────────────────────────

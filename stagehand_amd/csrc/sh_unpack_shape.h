@@ -42,12 +42,13 @@ constexpr uint32_t kThreads = SH_UNPACK_THREADS;
 constexpr uint32_t kUnrollI8 = SH_UNROLL_I8;
 constexpr uint32_t kUnrollF32 = SH_UNROLL_F32;
 constexpr uint32_t kChunkI8 = SH_CHUNK_I8;     // int8 elements per thread per chunk
-// Elements per 16-byte fp32 store: the dequant to fp32 and the widen move their tile in such steps,
-// lane-interleaved (sh_unpack.hip).
-constexpr uint32_t kStepI8F32 = 4;
-constexpr uint32_t kStepB16 = 4;
+// The dequant to fp32 and the widen move a thread's kPerThreadF32 elements in steps of one 16-byte
+// store, lane-interleaved (sh_unpack.hip). Two steps per thread: with four, a float32 double-stream
+// block of hidden 3072 (1.7 GB) took 318 us, with two 262 (6.5 TB/s), with one 356; one of hidden 1536 61.4, 60.6 and 62.8; a widen of
+// 1 G elements 1171, 997 (6.5 TB/s) and 1082.
+constexpr uint32_t kPerThreadF32 = 8;
+constexpr uint32_t kStepF32 = 4;
 constexpr uint32_t kChunkF32 = SH_CHUNK_F32;   // fp32 elements per thread per chunk (cast)
-constexpr uint32_t kChunkB16 = 16;             // bf16 elements per thread (widen), in steps of kStepB16
 // Byte kinds, per thread per chunk (measured on a 4 GiB region: copy 16 B
 // 6.57 TB/s vs 32 B 5.90 and 64 B 5.30; zero fill 32 B 6.29 TB/s vs 16 B 5.08
 // and 64 B 5.76).
@@ -63,19 +64,22 @@ static_assert(kChunkCopy % 16 == 0 && kChunkZero % 16 == 0, "byte chunks are who
 static_assert(kChunkI8 % 4 == 0 && kChunkF32 % 4 == 0, "chunks are whole 32-bit words");
 constexpr uint64_t kMaxDescElems = 1ull << 31;
 
+// Elements that stay together whatever the lead of a short region: a lead is a multiple of this.
 constexpr uint32_t chunk_of(uint32_t kind) {
   return (kind == SH_KIND_I8_ROWSCALE_BF16 || kind == SH_KIND_I8_ROWSCALE_F32) ? kChunkI8
          : kind == SH_KIND_F32_BF16                                              ? kChunkF32
-         : kind == SH_KIND_BF16_F32                                              ? kChunkB16
+         : kind == SH_KIND_BF16_F32                                              ? 16u
          : kind == SH_KIND_ZERO_BYTES                                            ? kChunkZero
                                                                                  : kChunkCopy;
 }
-constexpr uint32_t unroll_of(uint32_t kind) {
-  return (kind == SH_KIND_I8_ROWSCALE_BF16 || kind == SH_KIND_I8_ROWSCALE_F32) ? kUnrollI8
-         : kind == SH_KIND_F32_BF16                                              ? kUnrollF32
-                                                                                 : 1u;
+constexpr uint32_t per_thread(uint32_t kind) {
+  return kind == SH_KIND_I8_ROWSCALE_BF16                                  ? kUnrollI8 * kChunkI8
+         : kind == SH_KIND_F32_BF16                                        ? kUnrollF32 * kChunkF32
+         : (kind == SH_KIND_I8_ROWSCALE_F32 || kind == SH_KIND_BF16_F32) ? kPerThreadF32
+         : kind == SH_KIND_ZERO_BYTES                                      ? kChunkZero
+                                                                           : kChunkCopy;
 }
-constexpr uint32_t tile_of(uint32_t kind) { return kThreads * unroll_of(kind) * chunk_of(kind); }
+constexpr uint32_t tile_of(uint32_t kind) { return kThreads * per_thread(kind); }
 // Most tiles one plan may hold: a launch of n tiles has n * kThreads work-items, below 2^32.
 constexpr uint32_t kMaxTiles = 0xFFFFFFFFu / kThreads;
 

@@ -21,8 +21,8 @@ from stagehand_amd.unpack import (
 
 MIN_LEAD = 1 << 17
 # kind: (elements per tile, bytes of an output element)
-KINDS = {KIND_I8_ROWSCALE_BF16: (8192, 2), KIND_I8_ROWSCALE_F32: (8192, 4), KIND_F32_BF16: (2048, 2),
-         KIND_BF16_F32: (8192, 4)}
+KINDS = {KIND_I8_ROWSCALE_BF16: (8192, 2), KIND_I8_ROWSCALE_F32: (4096, 4), KIND_F32_BF16: (2048, 2),
+         KIND_BF16_F32: (4096, 4)}
 NO_LEAD = {KIND_COPY_BYTES: (8192, 1), KIND_ZERO_BYTES: (16384, 1)}
 
 
@@ -60,6 +60,23 @@ def test_a_lead_never_refuses_a_table_that_fits_without_it():
     lib = _native.lib()
     for rows, message in ((2064384, b"source"), (2064385, b"tiles")):  # fits: refused for its buffers alone
         table = make_descs([(KIND_F32_BF16, 0, 4098, rows, 2048, 0, 0)])
+        assert lib.sh_unpack_noalloc(table.ctypes.data, 1, None, 0, None, None, 0, None, 0,
+                                     None) == _native.SH_ERR_INVALID
+        assert message in lib.sh_last_error()
+
+
+def test_fp32_outputs_near_the_launch_limit_take_two_tiles_to_a_workgroup():
+    """A tile of an fp32 output is 4096 elements. A table of more tiles than a launch holds is built with
+    two to a workgroup, so that regions of up to 8192 elements per workgroup are accepted."""
+    max_tiles = (2**32 - 1) // 512
+    for kind in (KIND_I8_ROWSCALE_F32, KIND_BF16_F32):
+        assert tiles(kind, 0, 4096, rows=max_tiles) == max_tiles
+        assert tiles(kind, 0, 8192, rows=max_tiles) == max_tiles
+        with pytest.raises(ValueError, match="tiles"):
+            tiles(kind, 0, 8192, rows=max_tiles + 1)
+    lib = _native.lib()
+    for rows, message in ((2064384, b"source"), (2064385, b"tiles")):
+        table = make_descs([(KIND_BF16_F32, 0, 0, rows, 8192, 0, 0)])
         assert lib.sh_unpack_noalloc(table.ctypes.data, 1, None, 0, None, None, 0, None, 0,
                                      None) == _native.SH_ERR_INVALID
         assert message in lib.sh_last_error()
