@@ -230,8 +230,9 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 // HBM bounds this. Measured (MI355X; before, rows that were not back to back or not whole chunks
 // went element by element): a padded single-stream block of the 12B model with zero points 263 ->
 // 68 us (6.2 TB/s); 2999-wide rows 75 -> 65 us (6.2 TB/s) and a slab of 128 such tensors 1376 ->
-// 974 (1064 with its tiles off destination boundaries); the aligned double-stream block 159 -> 155 us (6.6 TB/s) and slab of 128 tensors 1010 -> 993
-// us (6.7 TB/s; 1001 before its ragged regions took the first tiles).
+// 974 (1064 with its tiles off destination boundaries); the aligned double-stream block 159 -> 155
+// us (6.6 TB/s) and slab of 128 tensors 1010 -> 993 (6.7 TB/s; 999 before its ragged regions took the
+// first tiles).
 //
 // ALONE: the kernel holds no other kind. Once a thread has all its loads, its stores go out back to
 // back, except for aligned rows in the kernel that holds no other kind: there each store waits for
