@@ -238,8 +238,8 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 // back, except for aligned rows in the kernel that holds no other kind: there each store waits for
 // the one before it. Measured, not paced against paced: double-stream block (mixed kernel) 154.9
 // against 157.5 us, padded block 68.1 against 70.3; but slab of 128 aligned tensors 1030-1060 against
-// 998-1007 us (6.6 GB, and 3% from 3 GB on; up to 2 GB the same). Pacing holds back writes in a stream that is two thirds writes; why only the aligned
-// long stream gains from it is not known.
+// 998-1007 us (6.6 GB, and 3% from 3 GB on; up to 2 GB the same). Pacing holds back writes in a
+// stream that is two thirds writes; why only the aligned long stream gains from it is not known.
 template <bool OUT_BF16, bool HAS_ZP, bool ALONE, uint32_t C, uint32_t U>
 __device__ __forceinline__ void i8_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel, uint32_t pad,
                                         const uint8_t* __restrict__ s, const float* __restrict__ sc,

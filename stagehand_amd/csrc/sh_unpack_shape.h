@@ -44,8 +44,8 @@ constexpr uint32_t kUnrollF32 = SH_UNROLL_F32;
 constexpr uint32_t kChunkI8 = SH_CHUNK_I8;     // int8 elements per thread per chunk
 // The dequant to fp32 and the widen move a thread's kPerThreadF32 elements in steps of one 16-byte
 // store, lane-interleaved (sh_unpack.hip). Two steps per thread: with four, a float32 double-stream
-// block of hidden 3072 (1.7 GB) took 318 us, with two 262 (6.5 TB/s), with one 356; one of hidden 1536 61.4, 60.6 and 62.8; a widen of
-// 1 G elements 1171, 997 (6.5 TB/s) and 1082.
+// block of hidden 3072 (1.7 GB) took 318 us, with two 266 (6.4 TB/s), with one 356; one of hidden
+// 1536 61.4, 60.6 and 62.8; a widen of 1 G elements 1171, 997 (6.5 TB/s) and 1082.
 constexpr uint32_t kPerThreadF32 = 8;
 constexpr uint32_t kStepF32 = 4;
 constexpr uint32_t kChunkF32 = SH_CHUNK_F32;   // fp32 elements per thread per chunk (cast)
