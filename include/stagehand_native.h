@@ -213,16 +213,16 @@ int sh_unpack_cast_f32_bf16(const sh_plan* plan,
  * (after splitting) and 32768 tiles is unpacked by one launch that reads it there. The launch
  * table and tile map of any other call go into a static device array of
  * SH_UNPACK_NOALLOC_SCRATCH_BYTES (8 MiB) in the library's code object, one per GPU it runs on,
- * held until sh_shutdown unloads the kernels (or the process ends). Limits: at most SH_UNPACK_NOALLOC_MAX_DESCS descriptors after the plan's
- * splitting of oversize regions and SH_UNPACK_NOALLOC_MAX_TILES tiles (config 2's dequant
- * needs 270k, its cast 1.08 M); beyond them it returns SH_ERR_INVALID. Calls that use the array
- * on one GPU share it and leave the last call's table in it. Each such call's kernels wait on the
- * device for the previous one's on that GPU (an event recorded after every such call), so calls
- * from several streams or threads do not corrupt each other. One made while `stream` is
- * being captured into a graph is not ordered that way (its kernels run at the graph's
- * replays): such replays must not overlap other such calls on that GPU. The first call on a GPU
- * loads the kernels there (as every entry point's first launch does) and, with the array, creates
- * the event. */
+ * held until sh_shutdown unloads the kernels (or the process ends). Limits: at most
+ * SH_UNPACK_NOALLOC_MAX_DESCS descriptors after the plan's splitting of oversize regions and
+ * SH_UNPACK_NOALLOC_MAX_TILES tiles (config 2's dequant needs 270k, its cast 1.08 M); beyond them
+ * it returns SH_ERR_INVALID. Each call's kernels, wherever its table is, wait on the device for
+ * the previous call's on that GPU (an event recorded after every call), so calls from several
+ * streams or threads neither corrupt a table nor overtake each other. A call made while `stream`
+ * is being captured into a graph is not ordered that way (its kernels run at the graph's replays):
+ * replays of a call that uses the array must not overlap other calls that use it on that GPU. The
+ * first call on a GPU loads the kernels there (as every entry point's first launch does) and
+ * creates the event. */
 #define SH_UNPACK_NOALLOC_MAX_DESCS 2048u
 #define SH_UNPACK_NOALLOC_MAX_TILES 2064384u
 #define SH_UNPACK_NOALLOC_SCRATCH_BYTES (8u << 20)

@@ -345,6 +345,30 @@ int launch_args(const sh_plan_info& in, const std::vector<sh_unpack_desc>& table
                            (hipStream_t)stream, args, who);
 }
 
+// Writes a checked table and its tile map into the scratch array at `base` and launches the unpack
+// kernel from there. `queued`: whether anything was launched, also when a later launch failed.
+int launch_scratch(const sh_plan_info& in, const std::vector<sh_unpack_desc>& table, void* base, const void* src,
+                   const float* scales, const float* zps, void* dst, void* stream, bool& queued, const char* who) {
+  const hipStream_t s = (hipStream_t)stream;
+  sh_unpack_desc* d_descs = (sh_unpack_desc*)base;
+  uint32_t* d_map = (uint32_t*)((uint8_t*)base + SH_UNPACK_NOALLOC_MAX_DESCS * sizeof(sh_unpack_desc));
+  const uint32_t nd = (uint32_t)table.size();
+  for (uint32_t first = 0; first < nd; first += kDescChunk) {
+    DescChunk c{};
+    c.first = first;
+    c.count = std::min(kDescChunk, nd - first);
+    std::copy(table.begin() + first, table.begin() + first + c.count, c.d);
+    void* args[] = {(void*)&c, (void*)&d_descs};
+    if (int st = sh::launch_kernel(sh::kKernPutDescs, 1, kDescChunk, s, args, who)) return st;
+    queued = true;
+  }
+  const sh_unpack_desc* table_arg = d_descs;
+  uint32_t tiles = in.n_tiles;
+  void* args[] = {(void*)&table_arg, (void*)&nd, (void*)&d_map, (void*)&tiles};
+  if (int st = sh::launch_kernel(sh::kKernFillTileMap, (in.n_tiles + 255) / 256, 256, s, args, who)) return st;
+  return launch_tiles(in, d_descs, d_map, src, scales, zps, dst, stream, who);
+}
+
 int launch(const sh_plan* plan, const void* src, size_t src_bytes, const float* scales,
            const float* zps, size_t n_scale, void* dst, size_t dst_bytes, void* stream,
            uint32_t required_mask, const char* who) {
@@ -367,16 +391,18 @@ int launch(const sh_plan* plan, const void* src, size_t src_bytes, const float* 
 // Most tiles of a launch whose table travels in its arguments. The search for a tile's descriptor
 // (five dependent scalar loads, against one of the tile map) costs every workgroup, the table and
 // tile map kernels cost the launch. Measured, arguments against scratch (MI355X, MLP and double-stream
-// blocks): 6 MB 9.5 against 15.2 us, 100 MB 16.0 and 25.3, 450 MB (18.5K tiles) 73.3 and 81.8, 1 GB
-// (41.5K tiles) 163.7 and about 163.
+// blocks): 6 MB 7.2-8.0 against 12.6 us, 100 MB 19.0 and 25.0, 450 MB (18.5K tiles) 67.9 and 74.0, 710
+// MB (28.9K tiles) 103.5 and 109.5, 2.8 GB (115K tiles) 461 and 458, 4.1 GB 668 and 658.
 constexpr uint32_t kMaxArgsTiles = 32768;
 
 // sh_unpack_noalloc's state. One lock orders the host side of every call; per device, an
 // event recorded after the last call's launches. Every call first makes its stream wait for
-// that event, so its writes to the device's scratch array start only after the previous call's
-// kernels have read it, whichever streams or threads the calls come from (on one stream the
-// wait costs nothing on the device). Nothing here has a destructor: the table is never freed (it
-// holds at most the largest plan seen) and the events end in sh_shutdown.
+// that event, whichever streams or threads the calls come from: a call that uses the device's
+// scratch array may write it only after the previous one's kernels have read it, and callers with
+// buffers in common rely on the order between any two calls, so a call whose table travels in its
+// arguments waits and records too (on one stream the wait costs nothing on the device). Nothing
+// here has a destructor: the table is never freed (it holds at most the largest plan seen) and the
+// events end in sh_shutdown.
 constexpr int kMaxDevices = 64;
 struct NoallocDevice {
   hipEvent_t done = nullptr;
@@ -428,8 +454,6 @@ extern "C" int sh_unpack_noalloc(const sh_unpack_desc* descs, uint32_t n, const 
                     (unsigned)SH_UNPACK_NOALLOC_MAX_TILES);
   if (in.n_tiles == 0) return SH_OK;
   if (int st = check_buffers(in, src, src_bytes, scales, n_scale, dst, dst_bytes, who)) return st;
-  if (table.size() <= kDescChunk && in.n_tiles <= kMaxArgsTiles)
-    return launch_args(in, table, src, scales, zero_points, dst, stream, who);
   int dev = -1;
   SH_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= kMaxDevices) return sh::fail(SH_ERR_INVALID, "%s: device %d out of range", who, dev);
@@ -445,27 +469,14 @@ extern "C" int sh_unpack_noalloc(const sh_unpack_desc* descs, uint32_t n, const 
   const bool eager = capture == hipStreamCaptureStatusNone;
   if (eager && nd_state.pending) SH_HIP(hipStreamWaitEvent(s, nd_state.done, 0));
 
-  sh_unpack_desc* d_descs = (sh_unpack_desc*)base;
-  uint32_t* d_map = (uint32_t*)((uint8_t*)base + SH_UNPACK_NOALLOC_MAX_DESCS * sizeof(sh_unpack_desc));
-  const uint32_t nd = (uint32_t)table.size();
   int st = SH_OK;
   bool queued = false;
-  for (uint32_t first = 0; first < nd && st == SH_OK; first += kDescChunk) {
-    DescChunk c{};
-    c.first = first;
-    c.count = std::min(kDescChunk, nd - first);
-    std::copy(table.begin() + first, table.begin() + first + c.count, c.d);
-    void* args[] = {(void*)&c, (void*)&d_descs};
-    st = sh::launch_kernel(sh::kKernPutDescs, 1, kDescChunk, s, args, who);
-    queued |= st == SH_OK;
+  if (table.size() <= kDescChunk && in.n_tiles <= kMaxArgsTiles) {
+    st = launch_args(in, table, src, scales, zero_points, dst, stream, who);
+    queued = st == SH_OK;
+  } else {
+    st = launch_scratch(in, table, base, src, scales, zero_points, dst, stream, queued, who);
   }
-  if (st == SH_OK) {
-    const sh_unpack_desc* table_arg = d_descs;
-    uint32_t tiles = in.n_tiles;
-    void* args[] = {(void*)&table_arg, (void*)&nd, (void*)&d_map, (void*)&tiles};
-    st = sh::launch_kernel(sh::kKernFillTileMap, (in.n_tiles + 255) / 256, 256, s, args, who);
-  }
-  if (st == SH_OK) st = launch_tiles(in, d_descs, d_map, src, scales, zero_points, dst, stream, who);
   if (eager && queued) {
     // Recorded after whatever was queued, also when a later launch failed: the next call must
     // not overwrite a table that a queued kernel may still read.

@@ -582,9 +582,8 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
 }
 
 // The launch table in the kernel's arguments: the descriptor of a tile is the last one whose
-// tile_begin is not above it. One launch in place of three, and no device array shared between calls:
-// an MLP block of 6 MB 9.5 us instead of 15.2, bound by the host's call (the rule and both sides are
-// at kMaxArgsTiles, sh_unpack.cpp).
+// tile_begin is not above it. One launch in place of three: an MLP block of 6 MB 7.2-8.0 us instead of
+// 12.6, bound by the host's call (the rule and both sides are at kMaxArgsTiles, sh_unpack.cpp).
 template <bool HAS_ZP>
 __device__ __forceinline__ void unpack_args_body(const DescArgs& a, const uint8_t* __restrict__ src,
                                                  const float* __restrict__ scales,

@@ -185,10 +185,10 @@ def unpack_noalloc(
     (``sh_unpack_noalloc``: a short table travels in the launch's arguments, a longer one lives in the
     library's static per-GPU scratch).
 
-    The results equal an :class:`UnpackPlan` of the same table run with ``sh_unpack``. Calls on one
-    GPU with tables of more than 32 descriptors or 32768 tiles share the scratch; each one's kernels
-    wait on the device for the previous one's, from any stream or thread. Such a call recorded into
-    a graph is not ordered that way: replays of the graph must not overlap others on that GPU."""
+    The results equal an :class:`UnpackPlan` of the same table run with ``sh_unpack``. Each call's
+    kernels wait on the device for the previous call's on that GPU, from any stream or thread. A
+    call recorded into a graph is not ordered that way; if its table has more than 32 descriptors or
+    32768 tiles, replays of the graph must not overlap other calls with such tables on that GPU."""
     table = np.ascontiguousarray(descs, dtype=DESC_DTYPE)
     sp, sb = _device_ptr(src, "src")
     dp, db = _device_ptr(dst, "dst")

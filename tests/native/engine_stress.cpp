@@ -15,6 +15,7 @@
 //   the host with its slot free, and the engine must go on working.
 // - VMM allocator: three threads take and release handles on eight regions under a ceiling of
 //   four while a fourth prefetches, changes priorities and reads statistics.
+// - Allocation-free unpack: calls on two streams, with short and long tables, keep their order.
 // Every byte that moves is checked; the sanitizers fail the run on a race, a use after free,
 // an out-of-bounds access or undefined behaviour.
 //
@@ -587,6 +588,49 @@ void vmm_stress(uint32_t seed, int iters) {
                refused.load(), (unsigned long long)st.evictions);
 }
 
+// ── allocation-free unpack: order of calls across streams ─────────────────
+
+// A call's kernels wait for the previous call's, whatever the streams and wherever the launch tables
+// travel (up to 32 regions in the launch's arguments, more in the scratch array): work behind a call
+// on one stream sees what was queued before the call before it on another. The kernels do nothing
+// here; the order is that of the copies around them.
+void noalloc_order() {
+  constexpr size_t kBig = 48u << 20;  // a copy long enough for an unordered one to overtake it
+  void *big_src = dmalloc(kBig), *big_dst = dmalloc(kBig), *out = dmalloc(64 * 16);
+  std::memset(big_src, 1, kBig);
+  std::vector<sh_unpack_desc> regions(40);
+  for (uint32_t i = 0; i < regions.size(); ++i) {
+    regions[i] = sh_unpack_desc{};
+    regions[i].dst_off = 16ull * i;
+    regions[i].rows = 1;
+    regions[i].cols = 16;
+    regions[i].kind = SH_KIND_ZERO_BYTES;
+  }
+  hipStream_t a = nullptr, b = nullptr;
+  check(hipStreamCreateWithFlags(&a, 0) == hipSuccess && hipStreamCreateWithFlags(&b, 0) == hipSuccess, "streams");
+  for (uint32_t first : {1u, 32u, 40u}) {
+    for (uint32_t second : {1u, 40u}) {
+      std::vector<uint8_t> before(1, 0), after(1, 0);
+      const uint8_t one = 1;
+      check(hipMemcpyAsync(big_dst, big_src, kBig, hipMemcpyDeviceToDevice, a) == hipSuccess, "copy");
+      check(hipMemcpyAsync(before.data(), &one, 1, hipMemcpyDeviceToDevice, a) == hipSuccess, "copy");
+      check(sh_unpack_noalloc(regions.data(), first, nullptr, 0, nullptr, nullptr, 0, out, 64 * 16, a) == SH_OK,
+            "sh_unpack_noalloc", first);
+      check(sh_unpack_noalloc(regions.data(), second, nullptr, 0, nullptr, nullptr, 0, out, 64 * 16, b) == SH_OK,
+            "sh_unpack_noalloc", second);
+      check(hipMemcpyAsync(after.data(), before.data(), 1, hipMemcpyDeviceToDevice, b) == hipSuccess, "copy");
+      check(hipStreamSynchronize(b) == hipSuccess, "sync");
+      check(after[0] == 1, "an allocation-free call waits for the one before it on another stream",
+            (long)(first * 100 + second));
+      check(hipStreamSynchronize(a) == hipSuccess, "sync");
+    }
+  }
+  check(hipStreamDestroy(a) == hipSuccess && hipStreamDestroy(b) == hipSuccess, "streams");
+  (void)hipFree(big_src);
+  (void)hipFree(big_dst);
+  (void)hipFree(out);
+}
+
 }  // namespace
 
 int main() {
@@ -611,6 +655,7 @@ int main() {
     for (std::thread& t : ts) t.join();
   }
   turbo_stress(5);
+  noalloc_order();
   check(sh_pool_destroy(pool) == SH_OK, "sh_pool_destroy");
   sh_live_counts live{};
   check(sh_shutdown(&live) == SH_OK, "sh_shutdown");

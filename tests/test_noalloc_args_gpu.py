@@ -1,6 +1,6 @@
 """``sh_unpack_noalloc`` around the limits of a table that travels in the launch's arguments (32
 descriptors, 32768 tiles): the same bytes as the plan-based entry point on both sides of them, on two
-streams at once, and at every replay of a captured call."""
+streams at once and in order across them, and at every replay of a captured call."""
 from __future__ import annotations
 
 import numpy as np
@@ -91,6 +91,33 @@ def test_short_and_long_tables_on_two_streams():
     for out in outs:
         for got, case in zip(out, cases):
             assert torch.equal(got, case[3])
+
+
+@pytest.mark.parametrize("first", [1, 32, 40])
+@pytest.mark.parametrize("second", [1, 40])
+def test_a_call_waits_for_the_one_before_it_on_another_stream(first, second):
+    """The second call reads what the first writes, on a stream of its own and with no other order
+    between them than the calls'. The first one's stream is busy for about a millisecond before."""
+    n = 40 * 4096
+    g = torch.Generator(device="cuda").manual_seed(first + second)
+    src = torch.randint(0, 256, (n,), dtype=torch.uint8, device="cuda", generator=g)
+    mid, out = torch.zeros_like(src), torch.zeros_like(src)
+    big = torch.zeros(2 << 30, dtype=torch.uint8, device="cuda")
+    busy = torch.empty_like(big)
+
+    def copies(regions: int):
+        each = n // regions
+        sizes = [each] * (regions - 1) + [n - each * (regions - 1)]
+        return make_descs([(KIND_COPY_BYTES, each * i, each * i, 1, size, 0, 0) for i, size in enumerate(sizes)])
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        busy.copy_(big)
+    unpack_noalloc(copies(first), src, mid, stream=a)
+    unpack_noalloc(copies(second), mid, out, stream=b)
+    torch.cuda.synchronize()
+    assert torch.equal(out, src)
 
 
 def test_captured_call_at_every_replay():
