@@ -182,9 +182,9 @@ int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool fewest, std::ve
   };
 
   // Regions of padded or ragged int8 rows take the first tiles: their workgroups run longer (chunks
-  // across rows are written twice), and last in the grid they would hold up its end. Measured, in
-  // front against in the caller's order: dequant slabs that end in 77-wide rows, 5 tensors 37.5 and
-  // 38.2 us, 20 tensors 158.3 and 159.7, 128 tensors 1001 and 1008.
+  // across rows need a second scale or are written twice), and last in the grid they would hold up its
+  // end. Measured, in front against in the caller's order: dequant slabs that end in 77-wide rows, 5
+  // tensors 36.9 and 37.3 us, 20 tensors 157.9 and 158.6, 128 tensors 992 and 995.
   for (const bool ragged_first : {true, false}) {
     for (uint32_t i = 0; i < n; ++i) {
       const sh_unpack_desc& d = descs[i];

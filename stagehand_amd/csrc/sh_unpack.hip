@@ -211,7 +211,8 @@ __device__ __forceinline__ bool whole_chunk(uint32_t e, uint32_t numel) {
 constexpr int kWaitVmcnt0 = 0x0F70;
 
 // Rows of at least a chunk, of any length and stride: a chunk lies in one row, or in the last `left`
-// elements of one row and the first C - left of the next.
+// elements of one row and the first C - left of the next. Narrow unpadded rows whose chunks cross
+// often take i8_narrow_rows instead.
 //
 // All chunks of a thread go through straight-line code as if each lay in one row with a finite
 // scale: the loads first, then the conversions and the stores. Only then are the exceptions seen
@@ -313,6 +314,57 @@ __device__ __forceinline__ void i8_rows(const sh_unpack_desc& d, uint32_t e0, ui
   }
 }
 
+// Unpadded rows of at least a chunk and below kNarrowRowBytes of output, where chunks cross rows: every
+// chunk takes its row's scale and the next one's (its own again where it ends inside the row) and is
+// written once. In such rows most wavefronts have a chunk across rows, and i8_rows' second pass over
+// them costs more than the second scale and the choice per element. As there, the loads go first,
+// without a branch, and the stores back to back once all of them are there.
+//
+// Measured (MI355X, one region; in brackets i8_rows, and the path before both, which tracked the row
+// element by element): 64 M elements to bf16, 9-wide rows 34.7 us [75, 34.6], 77 31.1 [47, 31.0], 255 30.7
+// [35.4, 30.6]; 1 G elements, 77 519 [934, 569], 513 510 [604, 560], 1023 509 [550, 559]; to fp32, 1 G elements, 9 995
+// [2163, 1352], 255 893 [904, 1340].
+template <bool OUT_BF16, bool HAS_ZP, uint32_t C, uint32_t U>
+__device__ __forceinline__ void i8_narrow_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel,
+                                               const uint8_t* __restrict__ s, const float* __restrict__ sc,
+                                               const float* __restrict__ zp, uint8_t* __restrict__ o) {
+  Words<C> q[U];
+  uint32_t row[U], left[U];
+  float s0[U], s1[U], z0[U], z1[U];
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    const uint32_t e = e0 + k * (kThreads * C);
+    const uint32_t i = whole_chunk<C>(e, numel) ? e : 0u;
+    row[k] = sh::udiv(i, d.div_magic);
+    left[k] = (row[k] + 1) * d.cols - i;  // modulo 2^32; the difference fits
+    q[k] = ldw<C>(s + i);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    const uint32_t next = left[k] < C ? row[k] + 1 : row[k];  // exists: the chunk lies below numel
+    s0[k] = sc[row[k]];
+    s1[k] = sc[next];
+    z0[k] = HAS_ZP ? zp[row[k]] : 0.0f;
+    z1[k] = HAS_ZP ? zp[next] : 0.0f;
+  }
+  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) {
+    const uint32_t e = e0 + k * (kThreads * C);
+    if (whole_chunk<C>(e, numel)) {
+      float se[C], ze[C];
+#pragma unroll
+      for (uint32_t j = 0; j < C; ++j) {
+        se[j] = j < left[k] ? s0[k] : s1[k];
+        ze[j] = j < left[k] ? z0[k] : z1[k];
+      }
+      dq_each_store<C, OUT_BF16, HAS_ZP>(q[k], se, ze, o + (size_t)e * (OUT_BF16 ? 2 : 4));
+    } else {
+      dq_edge<C, OUT_BF16, HAS_ZP>(d, e, numel, 0, s, sc, zp, o);
+    }
+  }
+}
+
 // Rows shorter than a chunk: the row is tracked element by element inside each chunk.
 template <bool OUT_BF16, bool HAS_ZP, uint32_t C, uint32_t U>
 __device__ __forceinline__ void i8_short_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel, uint32_t pad,
@@ -325,11 +377,22 @@ __device__ __forceinline__ void i8_short_rows(const sh_unpack_desc& d, uint32_t 
       uint32_t r = sh::udiv(e, d.div_magic);
       uint32_t c = e - r * d.cols;
       Words<C> q{};
-      if (pad == 0) q = ldw<C>(s + e);
+      if (pad == 0) {
+        q = ldw<C>(s + e);
+      } else {
+        uint32_t rq = r, cq = c;
+#pragma unroll
+        for (uint32_t j = 0; j < C; ++j) {
+          q.w[j / 4] |= (uint32_t)s[e + j + (uint64_t)rq * pad] << (8 * (j % 4));
+          if (++cq == d.cols) {
+            cq = 0;
+            ++rq;
+          }
+        }
+      }
       float se[C], ze[C];
 #pragma unroll
       for (uint32_t j = 0; j < C; ++j) {
-        if (pad != 0) q.w[j / 4] |= (uint32_t)s[e + j + (uint64_t)r * pad] << (8 * (j % 4));
         se[j] = sc[r];
         ze[j] = HAS_ZP ? zp[r] : 0.0f;
         if (++c == d.cols) {
@@ -343,6 +406,12 @@ __device__ __forceinline__ void i8_short_rows(const sh_unpack_desc& d, uint32_t 
     }
   }
 }
+
+// Output rows below this size take i8_narrow_rows where chunks cross rows. Above, fewer chunks cross, and
+// i8_rows is as fast or faster: rows of 1155 bf16 (64 M elements) 30.8 us against 30.4, (1 G) 518 and 509,
+// 3001 493 and 509, a slab of 128 tensors of 2999 to 11996 elements a row 966 and 1009; fp32, 700 822 and 833, a
+// double-stream block of hidden 3001 272 and 285.
+constexpr uint32_t kNarrowRowBytes = 2048;
 
 template <bool OUT_BF16, bool HAS_ZP, bool ALONE>
 __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
@@ -363,12 +432,16 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
   uint8_t* o = dst + d.dst_off;
   const float* sc = scales + d.scale_off;
   const float* zp = HAS_ZP ? zps + d.scale_off : nullptr;
+  const bool crossing = ((cols | d.lead) % C) != 0;  // chunks may lie across rows
+  const bool narrow = pad == 0 && crossing && cols >= C && cols < kNarrowRowBytes / (OUT_BF16 ? 2u : 4u);
   // A workgroup takes one tile, or two of an fp32 output where the table is near the launch limit.
   const uint32_t last = OUT_BF16 ? 0u : d.reserved;
   uint32_t e0 = (local << last) * T + threadIdx.x * C - d.lead;
 #pragma unroll 1
   for (uint32_t sub = 0; sub <= last; ++sub, e0 += T) {
-    if (cols >= C)
+    if (narrow)
+      i8_narrow_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, s, sc, zp, o);
+    else if (cols >= C)
       i8_rows<OUT_BF16, HAS_ZP, ALONE, C, U>(d, e0, numel, pad, s, sc, zp, o);
     else
       i8_short_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, pad, s, sc, zp, o);

@@ -2,9 +2,10 @@
 bit for bit, with canary bytes on both sides.
 
 The sizes sit where the kernels' paths meet: rows one element shorter, equal to and longer than a
-chunk (8 int8 to bf16, 4 to fp32), chunks that end exactly at a row's end, a source that ends with
-the last row's last element, and regions of one tile and one element more. Scales that make NaNs and
-infinities lie beside ordinary ones, in chunks of one row and of two.
+chunk (8 int8 to bf16, 4 to fp32), rows on both sides of 2 KiB of output (1024 bf16, 512 fp32), chunks
+that end exactly at a row's end, a source that ends with the last row's last element, and regions of
+one tile and one element more. Scales that make NaNs and infinities lie beside ordinary ones, in
+chunks of one row and of two.
 
 Regions just below and above 131072 elements: from there on the tiles of a dequant, cast or widen start
 on a destination boundary whatever the region's start, and its first chunk is cut."""
@@ -33,6 +34,10 @@ ROWS = [
     (300, 1, 0), (300, 1, 3), (200, 3, 1), (200, 4, 0), (200, 4, 5), (200, 5, 3), (90, 7, 2), (90, 8, 0), (90, 8, 8),
     (90, 9, 0), (90, 9, 7), (33, 1155, 0), (33, 1155, 16), (5, 4097, 1), (2, 8193, 0),
     (64, 2048, 16), (128, 1023, 0), (128, 1024, 0), (128, 1025, 3), (43, 3072, 0), (43, 3072, 4),
+    # the line between narrow and wide rows (2 KiB of output), and narrow rows of whole chunks in regions
+    # long enough to start on a boundary from any element, so that their chunks cross rows
+    (300, 511, 0), (300, 512, 0), (300, 513, 0), (2100, 64, 0), (8200, 16, 0), (16400, 8, 0), (32800, 4, 0), (160, 1016, 0),
+    (257, 511, 1),
 ]
 
 
