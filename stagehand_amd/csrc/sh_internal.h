@@ -78,7 +78,6 @@ enum KernelId : int {
   kKernDequantBf16 = 0,
   kKernDequantBf16Zp,
   kKernCastBf16,
-  kKernCastBf16Short,
   kKernMixed,
   kKernMixedZp,
   kKernUnpackArgs,

@@ -38,7 +38,6 @@ constexpr KernelSpec kKernelSpecs[sh::kKernelCount] = {
     {kModUnpack, "sh_dequant_i8_bf16_kernel"},
     {kModUnpack, "sh_dequant_i8_bf16_zp_kernel"},
     {kModUnpack, "sh_cast_f32_bf16_kernel"},
-    {kModUnpack, "sh_cast_f32_bf16_short_kernel"},
     {kModUnpack, "sh_unpack_mixed_kernel"},
     {kModUnpack, "sh_unpack_mixed_zp_kernel"},
     {kModUnpack, "sh_unpack_args_kernel"},

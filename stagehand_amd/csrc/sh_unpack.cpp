@@ -302,10 +302,6 @@ int check_buffers(const sh_plan_info& in, const void* src, size_t src_bytes, con
   return SH_OK;
 }
 
-// Most tiles of a cast that stores past the L2: 67 M elements, 400 MB moved (both sides measured at
-// tile_f32_bf16, sh_unpack.hip).
-constexpr uint32_t kShortCastTiles = 32768;
-
 // Launches the unpack kernel for a checked plan whose table and tile map are at d_descs /
 // d_tile_map on the current device.
 int launch_tiles(const sh_plan_info& in, const sh_unpack_desc* d_descs, const uint32_t* d_tile_map,
@@ -317,7 +313,7 @@ int launch_tiles(const sh_plan_info& in, const sh_unpack_desc* d_descs, const ui
   if (in.kind_mask == kMaskDequantBf16)
     kern = has_zp ? sh::kKernDequantBf16Zp : sh::kKernDequantBf16;
   else if (in.kind_mask == kMaskCastBf16)
-    kern = in.n_tiles <= kShortCastTiles ? sh::kKernCastBf16Short : sh::kKernCastBf16;
+    kern = sh::kKernCastBf16;
   else
     kern = has_zp ? sh::kKernMixedZp : sh::kKernMixed;
 

@@ -450,10 +450,10 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
 
 // ── fp32 → bf16 cast ──────────────────────────────────────────────────────
 
-// SHORT: a launch whose output the memory-side cache can hold a good part of; it stores past the L2
-// (nt) too. Measured (MI355X; plain against nt stores): 25 MB 5.2 and 4.9 us, 57 MB 12.5 and 10.5, 126
-// MB 24.5 and 22.5, 354 MB 61.6 and 59.4, 510 MB the same, 1 GB 165.0 and 165.8, 13 GB 2099 and 2158.
-template <bool SHORT>
+// Plain stores: the next kernel reads the output, and finds what the L2s still hold of it. Non-temporal
+// stores make a cast of up to 400 MB 4-10% faster by itself and the pair slower (MI355X, cast and a
+// matrix product that reads it, 64 rows: 2048x512 9.9 us with plain and 11.6 with nt stores, 3072x3072
+// 27.2 and 32.4, 8192x2048 30.2 and 39.1, 12288x3072 56.9 and 62.0).
 __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t local,
                                               const uint8_t* __restrict__ src,
                                               uint8_t* __restrict__ dst) {
@@ -477,10 +477,7 @@ __device__ __forceinline__ void tile_f32_bf16(const sh_unpack_desc& d, uint32_t 
 #pragma unroll
       for (uint32_t w = 0; w < C / 2; ++w)
         ow.w[w] = pack_hi(rne_hi_nan(__uint_as_float(v[k].w[2 * w])), rne_hi_nan(__uint_as_float(v[k].w[2 * w + 1])));
-      if constexpr (SHORT)
-        stw_nt<2 * C>(o + (size_t)e * 2, ow);
-      else
-        stw<2 * C>(o + (size_t)e * 2, ow);
+      stw<2 * C>(o + (size_t)e * 2, ow);
     } else {
 #pragma unroll 1
       for (uint32_t j = e; j != e + C; ++j) {  // cut by the region's start or end
@@ -600,7 +597,7 @@ __device__ __forceinline__ sh_unpack_desc load_desc(const sh_unpack_desc* __rest
   return d;
 }
 
-template <uint32_t MASK, bool HAS_ZP, bool SHORT>
+template <uint32_t MASK, bool HAS_ZP>
 __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t tile,
                                             const uint8_t* __restrict__ src,
                                             const float* __restrict__ scales,
@@ -614,7 +611,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
     return;
   }
   if constexpr (MASK == kMaskCastBf16) {
-    tile_f32_bf16<SHORT>(d, local, src, dst);
+    tile_f32_bf16(d, local, src, dst);
     return;
   }
   switch (d.kind) {
@@ -627,7 +624,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
         tile_i8<false, HAS_ZP, false>(d, local, src, scales, zps, dst);
       break;
     case SH_KIND_F32_BF16:
-      if constexpr ((MASK & bit(SH_KIND_F32_BF16)) != 0) tile_f32_bf16<SHORT>(d, local, src, dst);
+      if constexpr ((MASK & bit(SH_KIND_F32_BF16)) != 0) tile_f32_bf16(d, local, src, dst);
       break;
     case SH_KIND_BF16_F32:
       if constexpr ((MASK & bit(SH_KIND_BF16_F32)) != 0) tile_bf16_f32(d, local, src, dst);
@@ -643,7 +640,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
   }
 }
 
-template <uint32_t MASK, bool HAS_ZP, bool SHORT = false>
+template <uint32_t MASK, bool HAS_ZP>
 __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ descs,
                                             const uint32_t* __restrict__ tile_map,
                                             const uint8_t* __restrict__ src,
@@ -651,7 +648,7 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
                                             const float* __restrict__ zps,
                                             uint8_t* __restrict__ dst) {
   const uint32_t tile = blockIdx.x;
-  unpack_tile<MASK, HAS_ZP, SHORT>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
+  unpack_tile<MASK, HAS_ZP>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
 }
 
 // The launch table in the kernel's arguments: the descriptor of a tile is the last one whose
@@ -667,7 +664,7 @@ __device__ __forceinline__ void unpack_args_body(const DescArgs& a, const uint8_
 #pragma unroll
   for (uint32_t step = kDescChunk / 2; step > 0; step /= 2)
     if (a.tile_begin[i + step] <= tile) i += step;
-  unpack_tile<kMaskAll, HAS_ZP, true>(load_desc(a.d + i), tile, src, scales, zps, dst);
+  unpack_tile<kMaskAll, HAS_ZP>(load_desc(a.d + i), tile, src, scales, zps, dst);
 }
 
 }  // namespace
@@ -685,9 +682,6 @@ extern "C" __global__ __launch_bounds__(kThreads) void sh_dequant_i8_bf16_zp_ker
 }
 extern "C" __global__ __launch_bounds__(kThreads) void sh_cast_f32_bf16_kernel(SH_KERNEL_ARGS) {
   unpack_body<kMaskCastBf16, false>(descs, tile_map, src, scales, zps, dst);
-}
-extern "C" __global__ __launch_bounds__(kThreads) void sh_cast_f32_bf16_short_kernel(SH_KERNEL_ARGS) {
-  unpack_body<kMaskCastBf16, false, true>(descs, tile_map, src, scales, zps, dst);
 }
 extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_kernel(SH_KERNEL_ARGS) {
   unpack_body<kMaskAll, false>(descs, tile_map, src, scales, zps, dst);

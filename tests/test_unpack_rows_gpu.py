@@ -110,9 +110,9 @@ def test_flat_regions_from_any_start(numel, start):
 
 
 @pytest.mark.parametrize("numel", [2048 * 32768, 2048 * 32768 + 1])
-def test_cast_on_both_sides_of_the_kernel_choice(numel):
-    """A cast-only plan takes another kernel above 32768 tiles of 2048 elements; torch's device cast
-    rounds the same way (no NaN here)."""
+def test_cast_of_whole_tiles_and_one_element_more(numel):
+    """A cast-only plan of whole tiles of 2048 elements and of one element more; torch's device cast rounds
+    the same way (no NaN here)."""
     g = torch.Generator(device="cuda").manual_seed(numel)
     src = torch.randn(numel, device="cuda", generator=g)
     dst = torch.empty(numel, dtype=torch.bfloat16, device="cuda")
