@@ -96,8 +96,9 @@ int launch_block_changed(const void* buf, uint64_t bytes, uint32_t chunk_bytes, 
   uint64_t chunk = chunk_bytes;
   const uint64_t n = chunks_of(bytes, chunk_bytes);
   void* args[] = {(void*)&b, (void*)&bytes, (void*)&chunk, (void*)&digests, (void*)&changed};
-  return launch_kernel(kKernDigestCompare, (uint32_t)n, threads_for(n, bytes, chunk_bytes), stream, args,
-                       "sh_block_changed");
+  const uint32_t threads = threads_for(n, bytes, chunk_bytes);
+  return launch_kernel(threads == kDigestThreads ? kKernDigestCompare : kKernDigestCompareWide, (uint32_t)n, threads,
+                       stream, args, "sh_block_changed");
 }
 
 int launch_block_digest(const void* buf, uint64_t bytes, uint32_t chunk_bytes, uint64_t* digests,
@@ -108,7 +109,9 @@ int launch_block_digest(const void* buf, uint64_t bytes, uint32_t chunk_bytes, u
   uint64_t chunk = chunk_bytes;
   const uint64_t n = chunks_of(bytes, chunk_bytes);
   void* args[] = {(void*)&b, (void*)&bytes, (void*)&chunk, (void*)&digests};
-  return launch_kernel(kKernDigest, (uint32_t)n, threads_for(n, bytes, chunk_bytes), stream, args, "sh_block_digest");
+  const uint32_t threads = threads_for(n, bytes, chunk_bytes);
+  return launch_kernel(threads == kDigestThreads ? kKernDigest : kKernDigestWide, (uint32_t)n, threads, stream, args,
+                       "sh_block_digest");
 }
 
 }  // namespace sh

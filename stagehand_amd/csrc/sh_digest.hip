@@ -10,11 +10,11 @@
 
 namespace {
 
-// One workgroup per chunk, of any number of whole wavefronts up to kDigestMaxThreads (threads_for,
-// sh_digest.cpp, chooses). COMPARE: changed[c] = 1 when the chunk's digest differs from
+// One workgroup per chunk. COMPARE: changed[c] = 1 when the chunk's digest differs from
 // digests[2c], digests[2c + 1], else 0; otherwise the digest is written there.
-// THREADS: the workgroup size where it is known when compiled (the loop of the long launches'
-// workgroups is 1-2% faster so), else 0.
+// THREADS: the workgroup size where it is known when compiled, else 0: any number of whole wavefronts
+// up to kDigestMaxThreads (threads_for, sh_digest.cpp, chooses). Compiled for 768, which the longest
+// launches take, the loop is no faster (2960 chunks of 256 KiB 115 us both ways).
 template <bool COMPARE, uint32_t THREADS>
 __device__ __forceinline__ void digest_body(const uint8_t* __restrict__ buf, uint64_t bytes, uint64_t chunk,
                                             uint64_t* __restrict__ digests, uint8_t* __restrict__ changed) {
@@ -70,19 +70,28 @@ __device__ __forceinline__ void digest_body(const uint8_t* __restrict__ buf, uin
 
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(kDigestMaxThreads) void sh_digest_kernel(
-    const uint8_t* __restrict__ buf, uint64_t bytes, uint64_t chunk, uint64_t* __restrict__ digests) {
-  if (blockDim.x == kDigestThreads)
-    digest_body<false, kDigestThreads>(buf, bytes, chunk, digests, nullptr);
-  else
-    digest_body<false, 0>(buf, bytes, chunk, digests, nullptr);
+// Workgroups of kDigestThreads have kernels of their own: one kernel that tests the workgroup's size
+// took 3% longer for short launches of small chunks (1 to 1024 chunks of 16 KiB 3.7-5.3 us against
+// 3.6-5.2).
+extern "C" __global__ __launch_bounds__(kDigestThreads) void sh_digest_kernel(const uint8_t* __restrict__ buf,
+                                                                              uint64_t bytes, uint64_t chunk,
+                                                                              uint64_t* __restrict__ digests) {
+  digest_body<false, kDigestThreads>(buf, bytes, chunk, digests, nullptr);
 }
 
-extern "C" __global__ __launch_bounds__(kDigestMaxThreads) void sh_digest_compare_kernel(
+extern "C" __global__ __launch_bounds__(kDigestThreads) void sh_digest_compare_kernel(
     const uint8_t* __restrict__ buf, uint64_t bytes, uint64_t chunk, const uint64_t* __restrict__ digests,
     uint8_t* __restrict__ changed) {
-  if (blockDim.x == kDigestThreads)
-    digest_body<true, kDigestThreads>(buf, bytes, chunk, const_cast<uint64_t*>(digests), changed);
-  else
-    digest_body<true, 0>(buf, bytes, chunk, const_cast<uint64_t*>(digests), changed);
+  digest_body<true, kDigestThreads>(buf, bytes, chunk, const_cast<uint64_t*>(digests), changed);
+}
+
+extern "C" __global__ __launch_bounds__(kDigestMaxThreads) void sh_digest_wide_kernel(
+    const uint8_t* __restrict__ buf, uint64_t bytes, uint64_t chunk, uint64_t* __restrict__ digests) {
+  digest_body<false, 0>(buf, bytes, chunk, digests, nullptr);
+}
+
+extern "C" __global__ __launch_bounds__(kDigestMaxThreads) void sh_digest_compare_wide_kernel(
+    const uint8_t* __restrict__ buf, uint64_t bytes, uint64_t chunk, const uint64_t* __restrict__ digests,
+    uint8_t* __restrict__ changed) {
+  digest_body<true, 0>(buf, bytes, chunk, const_cast<uint64_t*>(digests), changed);
 }

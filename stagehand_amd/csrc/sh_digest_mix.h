@@ -10,7 +10,9 @@
 namespace {
 
 constexpr uint32_t kKey = 0x9E3779B9u;  // word j's key is j * kKey mod 2^32
-constexpr uint32_t kDigestThreads = 256;  // work-items per chunk of a long launch
+// Work-items per chunk: kDigestThreads, or more (up to kDigestMaxThreads) where the number of chunks or
+// their size leaves compute units idle (threads_for, sh_digest.cpp).
+constexpr uint32_t kDigestThreads = 256;
 constexpr uint32_t kDigestMaxThreads = 1024;
 
 // MurmurHash3's 32-bit finalizer (Austin Appleby, public domain).

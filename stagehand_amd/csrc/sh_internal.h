@@ -85,7 +85,9 @@ enum KernelId : int {
   kKernPutDescs,
   kKernFillTileMap,
   kKernDigest,
+  kKernDigestWide,
   kKernDigestCompare,
+  kKernDigestCompareWide,
   kKernelCount
 };
 // Launches kernel `id` of the current device: a 1-D grid of `grid` workgroups of `block`

@@ -45,7 +45,9 @@ constexpr KernelSpec kKernelSpecs[sh::kKernelCount] = {
     {kModUnpack, "sh_put_descs_kernel"},
     {kModUnpack, "sh_fill_tile_map_kernel"},
     {kModDigest, "sh_digest_kernel"},
+    {kModDigest, "sh_digest_wide_kernel"},
     {kModDigest, "sh_digest_compare_kernel"},
+    {kModDigest, "sh_digest_compare_wide_kernel"},
 };
 
 struct DeviceKernels {

@@ -418,13 +418,13 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned int gx, unsigned int,
   if (should_fail("hipModuleLaunchKernel")) return hipErrorLaunchFailure;
   const std::string& name = reinterpret_cast<FakeFunction*>(f)->name;
   if (gx == 0) return hipErrorInvalidConfiguration;
-  if (name == "sh_digest_kernel") {
+  if (name == "sh_digest_kernel" || name == "sh_digest_wide_kernel") {
     const uint8_t* buf = *(const uint8_t**)params[0];
     const uint64_t bytes = *(const uint64_t*)params[1];
     const uint64_t chunk = *(const uint64_t*)params[2];
     uint64_t* digests = *(uint64_t**)params[3];
     stream_of(s)->push([=] { (void)sh_block_digest_host(buf, bytes, (uint32_t)chunk, digests); });
-  } else if (name == "sh_digest_compare_kernel") {
+  } else if (name == "sh_digest_compare_kernel" || name == "sh_digest_compare_wide_kernel") {
     const uint8_t* buf = *(const uint8_t**)params[0];
     const uint64_t bytes = *(const uint64_t*)params[1];
     const uint64_t chunk = *(const uint64_t*)params[2];
