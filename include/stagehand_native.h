@@ -210,7 +210,7 @@ int sh_unpack_cast_f32_bf16(const sh_plan* plan,
  * sh_plan_create + sh_unpack + sh_plan_destroy do for `descs`, with the same kernels and the
  * same results, but it calls no device allocator. Descriptors reach the device as kernel
  * arguments, so nothing on the host has to outlive the call: a table of at most 32 descriptors
- * (after splitting) and 32768 tiles is unpacked by one launch that reads it there. The launch
+ * (after splitting) and 49152 tiles is unpacked by one launch that reads it there. The launch
  * table and tile map of any other call go into a static device array of
  * SH_UNPACK_NOALLOC_SCRATCH_BYTES (8 MiB) in the library's code object, one per GPU it runs on,
  * held until sh_shutdown unloads the kernels (or the process ends). Limits: at most

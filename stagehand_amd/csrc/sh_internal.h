@@ -80,6 +80,8 @@ enum KernelId : int {
   kKernCastBf16,
   kKernMixed,
   kKernMixedZp,
+  kKernMixedPaced,
+  kKernMixedPacedZp,
   kKernUnpackArgs,
   kKernUnpackArgsZp,
   kKernPutDescs,

@@ -40,6 +40,8 @@ constexpr KernelSpec kKernelSpecs[sh::kKernelCount] = {
     {kModUnpack, "sh_cast_f32_bf16_kernel"},
     {kModUnpack, "sh_unpack_mixed_kernel"},
     {kModUnpack, "sh_unpack_mixed_zp_kernel"},
+    {kModUnpack, "sh_unpack_mixed_paced_kernel"},
+    {kModUnpack, "sh_unpack_mixed_paced_zp_kernel"},
     {kModUnpack, "sh_unpack_args_kernel"},
     {kModUnpack, "sh_unpack_args_zp_kernel"},
     {kModUnpack, "sh_put_descs_kernel"},

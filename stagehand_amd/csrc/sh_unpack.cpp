@@ -303,8 +303,8 @@ int check_buffers(const sh_plan_info& in, const void* src, size_t src_bytes, con
 }
 
 // Launches the unpack kernel for a checked plan whose table and tile map are at d_descs /
-// d_tile_map on the current device.
-int launch_tiles(const sh_plan_info& in, const sh_unpack_desc* d_descs, const uint32_t* d_tile_map,
+// d_tile_map on the current device. paced: the mixed kernel that paces aligned dequant rows (i8_rows).
+int launch_tiles(const sh_plan_info& in, const sh_unpack_desc* d_descs, const uint32_t* d_tile_map, bool paced,
                  const void* src, const float* scales, const float* zps, void* dst, void* stream, const char* who) {
   const bool has_i8 = (in.kind_mask & (bit(SH_KIND_I8_ROWSCALE_BF16) | bit(SH_KIND_I8_ROWSCALE_F32))) != 0;
   const bool has_zp = has_i8 && zps != nullptr;
@@ -314,6 +314,8 @@ int launch_tiles(const sh_plan_info& in, const sh_unpack_desc* d_descs, const ui
     kern = has_zp ? sh::kKernDequantBf16Zp : sh::kKernDequantBf16;
   else if (in.kind_mask == kMaskCastBf16)
     kern = sh::kKernCastBf16;
+  else if (paced)
+    kern = has_zp ? sh::kKernMixedPacedZp : sh::kKernMixedPaced;
   else
     kern = has_zp ? sh::kKernMixedZp : sh::kKernMixed;
 
@@ -341,6 +343,12 @@ int launch_args(const sh_plan_info& in, const std::vector<sh_unpack_desc>& table
                            (hipStream_t)stream, args, who);
 }
 
+// Most tiles of a mixed table in the scratch array whose aligned dequant rows are not paced (i8_rows). Not paced
+// against paced (double-stream blocks): 41.5K tiles 168.7 and 169.8 us, 56.5K 232.0 and 229.6, 74K 300.8 and
+// 296.3, 115K 458.0 and 444.6, 166K 660.9 and 631.2 (before rows of any length moved to whole chunks
+// 167.5, 228.0, 294.8, 446.5 and 635.3).
+constexpr uint32_t kMaxUnpacedTiles = 49152;
+
 // Writes a checked table and its tile map into the scratch array at `base` and launches the unpack
 // kernel from there. `queued`: whether anything was launched, also when a later launch failed.
 int launch_scratch(const sh_plan_info& in, const std::vector<sh_unpack_desc>& table, void* base, const void* src,
@@ -362,7 +370,7 @@ int launch_scratch(const sh_plan_info& in, const std::vector<sh_unpack_desc>& ta
   uint32_t tiles = in.n_tiles;
   void* args[] = {(void*)&table_arg, (void*)&nd, (void*)&d_map, (void*)&tiles};
   if (int st = sh::launch_kernel(sh::kKernFillTileMap, (in.n_tiles + 255) / 256, 256, s, args, who)) return st;
-  return launch_tiles(in, d_descs, d_map, src, scales, zps, dst, stream, who);
+  return launch_tiles(in, d_descs, d_map, in.n_tiles > kMaxUnpacedTiles, src, scales, zps, dst, stream, who);
 }
 
 int launch(const sh_plan* plan, const void* src, size_t src_bytes, const float* scales,
@@ -381,15 +389,15 @@ int launch(const sh_plan* plan, const void* src, size_t src_bytes, const float* 
     return sh::fail(SH_ERR_INVALID, "%s: plan was built on device %d but device %d is current", who,
                     plan->device, cur);
   if (int st = check_buffers(in, src, src_bytes, scales, n_scale, dst, dst_bytes, who)) return st;
-  return launch_tiles(in, plan->d_descs, plan->d_tile_map, src, scales, zps, dst, stream, who);
+  return launch_tiles(in, plan->d_descs, plan->d_tile_map, false, src, scales, zps, dst, stream, who);
 }
 
 // Most tiles of a launch whose table travels in its arguments. The search for a tile's descriptor
 // (five dependent scalar loads, against one of the tile map) costs every workgroup, the table and
 // tile map kernels cost the launch. Measured, arguments against scratch (MI355X, MLP and double-stream
-// blocks): 6 MB 7.2-8.0 against 12.6 us, 100 MB 19.0 and 25.0, 450 MB (18.5K tiles) 67.9 and 74.0, 710
-// MB (28.9K tiles) 103.5 and 109.5, 2.8 GB (115K tiles) 461 and 458, 4.1 GB 668 and 658.
-constexpr uint32_t kMaxArgsTiles = 32768;
+// blocks): 6 MB 7.2-8.0 against 12.6 us, 100 MB 19.0 and 25.0, 450 MB (18.5K tiles) 67.9 and 74.0, 1 GB
+// (41.5K tiles) 164.3 and 168.2, 1.2 GB (48.7K) 195.8 and 199.6, 1.8 GB (73.8K) 295.1 and 292.8.
+constexpr uint32_t kMaxArgsTiles = 49152;
 
 // sh_unpack_noalloc's state. One lock orders the host side of every call; per device, an
 // event recorded after the last call's launches. Every call first makes its stream wait for

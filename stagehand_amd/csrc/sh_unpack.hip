@@ -235,13 +235,14 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 // us (6.6 TB/s) and slab of 128 tensors 1010 -> 993 (6.7 TB/s; 999 before its ragged regions took the
 // first tiles).
 //
-// ALONE: the kernel holds no other kind. Once a thread has all its loads, its stores go out back to
-// back, except for aligned rows in the kernel that holds no other kind: there each store waits for
-// the one before it. Measured, not paced against paced: double-stream block (mixed kernel) 154.9
-// against 157.5 us, padded block 68.1 against 70.3; but slab of 128 aligned tensors 1030-1060 against
-// 998-1007 us (6.6 GB, and 3% from 3 GB on; up to 2 GB the same). Pacing holds back writes in a
-// stream that is two thirds writes; why only the aligned long stream gains from it is not known.
-template <bool OUT_BF16, bool HAS_ZP, bool ALONE, uint32_t C, uint32_t U>
+// Once a thread has all its loads, its stores go out back to back, except (PACED) for aligned rows in
+// the kernel that holds no other kind and in the one for long tables of sh_unpack_noalloc: there each
+// store waits for the one before it. Measured, not paced against paced: double-stream block (mixed
+// kernel) 154.9 against 157.5 us, padded block 68.1 against 70.3; but slab of 128 aligned tensors 1030-1060
+// against 998-1007 us (6.6 GB, and 3% from 3 GB on; up to 2 GB the same), and a mixed table in the scratch
+// array of 74K tiles 300.8 against 296.3, of 166K 660.9 against 631.2. Pacing holds back writes in a stream
+// that is two thirds writes; why only these gain from it is not known.
+template <bool OUT_BF16, bool HAS_ZP, bool PACED, uint32_t C, uint32_t U>
 __device__ __forceinline__ void i8_rows(const sh_unpack_desc& d, uint32_t e0, uint32_t numel, uint32_t pad,
                                         const uint8_t* __restrict__ s, const float* __restrict__ sc,
                                         const float* __restrict__ zp, uint8_t* __restrict__ o) {
@@ -261,7 +262,7 @@ __device__ __forceinline__ void i8_rows(const sh_unpack_desc& d, uint32_t e0, ui
     sv[k] = sc[row[k]];
     zv[k] = HAS_ZP ? zp[row[k]] : 0.0f;
   }
-  if (ALONE && pad == 0 && (d.cols % C) == 0 && (d.lead % C) == 0) {
+  if (PACED && pad == 0 && (d.cols % C) == 0 && (d.lead % C) == 0) {
 #pragma unroll
     for (uint32_t k = 0; k < U; ++k) {
       const uint32_t e = e0 + k * (kThreads * C);
@@ -413,7 +414,7 @@ __device__ __forceinline__ void i8_short_rows(const sh_unpack_desc& d, uint32_t 
 // double-stream block of hidden 3001 272 and 285.
 constexpr uint32_t kNarrowRowBytes = 2048;
 
-template <bool OUT_BF16, bool HAS_ZP, bool ALONE>
+template <bool OUT_BF16, bool HAS_ZP, bool PACED>
 __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
                                         const uint8_t* __restrict__ src,
                                         const float* __restrict__ scales,
@@ -442,7 +443,7 @@ __device__ __forceinline__ void tile_i8(const sh_unpack_desc& d, uint32_t local,
     if (narrow)
       i8_narrow_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, s, sc, zp, o);
     else if (cols >= C)
-      i8_rows<OUT_BF16, HAS_ZP, ALONE, C, U>(d, e0, numel, pad, s, sc, zp, o);
+      i8_rows<OUT_BF16, HAS_ZP, PACED, C, U>(d, e0, numel, pad, s, sc, zp, o);
     else
       i8_short_rows<OUT_BF16, HAS_ZP, C, U>(d, e0, numel, pad, s, sc, zp, o);
   }
@@ -597,7 +598,7 @@ __device__ __forceinline__ sh_unpack_desc load_desc(const sh_unpack_desc* __rest
   return d;
 }
 
-template <uint32_t MASK, bool HAS_ZP>
+template <uint32_t MASK, bool HAS_ZP, bool PACED>
 __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t tile,
                                             const uint8_t* __restrict__ src,
                                             const float* __restrict__ scales,
@@ -617,7 +618,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
   switch (d.kind) {
     case SH_KIND_I8_ROWSCALE_BF16:
       if constexpr ((MASK & bit(SH_KIND_I8_ROWSCALE_BF16)) != 0)
-        tile_i8<true, HAS_ZP, false>(d, local, src, scales, zps, dst);
+        tile_i8<true, HAS_ZP, PACED>(d, local, src, scales, zps, dst);
       break;
     case SH_KIND_I8_ROWSCALE_F32:
       if constexpr ((MASK & bit(SH_KIND_I8_ROWSCALE_F32)) != 0)
@@ -640,7 +641,7 @@ __device__ __forceinline__ void unpack_tile(const sh_unpack_desc& d, uint32_t ti
   }
 }
 
-template <uint32_t MASK, bool HAS_ZP>
+template <uint32_t MASK, bool HAS_ZP, bool PACED = false>
 __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ descs,
                                             const uint32_t* __restrict__ tile_map,
                                             const uint8_t* __restrict__ src,
@@ -648,7 +649,7 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
                                             const float* __restrict__ zps,
                                             uint8_t* __restrict__ dst) {
   const uint32_t tile = blockIdx.x;
-  unpack_tile<MASK, HAS_ZP>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
+  unpack_tile<MASK, HAS_ZP, PACED>(load_desc(descs + tile_map[tile]), tile, src, scales, zps, dst);
 }
 
 // The launch table in the kernel's arguments: the descriptor of a tile is the last one whose
@@ -664,7 +665,7 @@ __device__ __forceinline__ void unpack_args_body(const DescArgs& a, const uint8_
 #pragma unroll
   for (uint32_t step = kDescChunk / 2; step > 0; step /= 2)
     if (a.tile_begin[i + step] <= tile) i += step;
-  unpack_tile<kMaskAll, HAS_ZP>(load_desc(a.d + i), tile, src, scales, zps, dst);
+  unpack_tile<kMaskAll, HAS_ZP, false>(load_desc(a.d + i), tile, src, scales, zps, dst);
 }
 
 }  // namespace
@@ -688,6 +689,13 @@ extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_kernel(SH
 }
 extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_zp_kernel(SH_KERNEL_ARGS) {
   unpack_body<kMaskAll, true>(descs, tile_map, src, scales, zps, dst);
+}
+
+extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_paced_kernel(SH_KERNEL_ARGS) {
+  unpack_body<kMaskAll, false, true>(descs, tile_map, src, scales, zps, dst);
+}
+extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_mixed_paced_zp_kernel(SH_KERNEL_ARGS) {
+  unpack_body<kMaskAll, true, true>(descs, tile_map, src, scales, zps, dst);
 }
 
 extern "C" __global__ __launch_bounds__(kThreads) void sh_unpack_args_kernel(

@@ -188,7 +188,7 @@ def unpack_noalloc(
     The results equal an :class:`UnpackPlan` of the same table run with ``sh_unpack``. Each call's
     kernels wait on the device for the previous call's on that GPU, from any stream or thread. A
     call recorded into a graph is not ordered that way; if its table has more than 32 descriptors or
-    32768 tiles, replays of the graph must not overlap other calls with such tables on that GPU."""
+    49152 tiles, replays of the graph must not overlap other calls with such tables on that GPU."""
     table = np.ascontiguousarray(descs, dtype=DESC_DTYPE)
     sp, sb = _device_ptr(src, "src")
     dp, db = _device_ptr(dst, "dst")

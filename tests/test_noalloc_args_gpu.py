@@ -1,5 +1,5 @@
 """``sh_unpack_noalloc`` around the limits of a table that travels in the launch's arguments (32
-descriptors, 32768 tiles): the same bytes as the plan-based entry point on both sides of them, on two
+descriptors, 49152 tiles): the same bytes as the plan-based entry point on both sides of them, on two
 streams at once and in order across them, and at every replay of a captured call."""
 from __future__ import annotations
 
@@ -65,13 +65,28 @@ def test_tables_on_both_sides_of_the_argument_limit(n, zp):
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("tiles", [32768, 32769])
+@pytest.mark.parametrize("tiles", [32768, 32769, 49152, 49153])
 def test_tile_limit_of_the_arguments(tiles):
     n = 8192 * tiles
     src = torch.arange(n // 8, device="cuda").view(torch.uint8)
     got = torch.zeros_like(src)
     unpack_noalloc(make_descs([(KIND_COPY_BYTES, 0, 0, 1, n, 0, 0)]), src, got)
     assert torch.equal(got, src)
+
+
+@pytest.mark.parametrize("zp", [False, True])
+def test_long_table_of_several_kinds(zp):
+    """More tiles than the arguments take, of aligned int8 rows between a copy and a short odd region."""
+    rows, cols = 49160, 8192
+    descs = make_descs([(KIND_COPY_BYTES, 0, 0, 1, 1001, 0, 0), (KIND_I8_ROWSCALE_BF16, 1001, 1002, rows, cols, 0, 0),
+                        (KIND_I8_ROWSCALE_BF16, 1001 + rows * cols, 1002 + 2 * rows * cols, 7, 333, 0, rows)])
+    n_scale = rows + 7
+    src, scales, zps = _inputs(1001 + rows * cols + 7 * 333, n_scale, 5)
+    dst_bytes = 1002 + 2 * rows * cols + 2 * 7 * 333
+    want = _want(descs, src, dst_bytes, scales, zps if zp else None)
+    got = torch.full_like(want, 0xA5)
+    unpack_noalloc(descs, src, got, scales, zps if zp else None)
+    assert torch.equal(got, want)
 
 
 def test_short_and_long_tables_on_two_streams():
