@@ -51,7 +51,8 @@ uint64_t chunks_of(uint64_t bytes, uint32_t chunk_bytes) {
 }
 
 // Work-items of each chunk's workgroup, by the number of chunks (MI355X: 256 compute units, each with
-// room for 28 wavefronts of these kernels' registers).
+// room for 28 wavefronts of these kernels' registers; a partition of the chip has fewer, and gets the
+// sizes of the whole one: the same digests, at times not the fastest size).
 // - Fewer chunks than compute units: each chunk has a compute unit to itself and its mixing takes all
 //   of its vector ALU, so the more wavefronts hide each other's latency the better. 49 chunks of 256
 //   KiB (digest and comparison) 21.6 us with 1024, 23.6 with 512, 34.3 with 256 work-items; 16 chunks

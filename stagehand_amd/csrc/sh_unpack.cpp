@@ -50,7 +50,7 @@ uint32_t dst_elem_bytes(uint32_t kind) {
 
 // Elements placed before element 0 in a descriptor's first tile, so that the tiles' destination
 // spans start on kDstAlign-byte boundaries of the destination buffer (whose base the caller's
-// allocator aligns to at least that), or failing that on 64-byte lines. Measured on MI355X:
+// allocator aligns to at least that). Measured on MI355X:
 // - a region that starts inside a 64-byte line has every wavefront write a partial line at both
 //   ends, shared with the neighbouring wavefront, often on another XCD; a 2.2 G-element dequant
 //   region whose destination started 16 or 32 bytes into a line ran 1.9% slower, a cast 1.2%;
@@ -63,12 +63,12 @@ uint32_t dst_elem_bytes(uint32_t kind) {
 // are whole chunks, inside one row, so any region gets one. Another lead cuts the region's first
 // chunk (written element by element) and makes int8 chunks cross rows, so only a dequant, cast
 // or widen of kMinRaggedLead elements or more gets one: 16 tiles of dequant, of which it adds at
-// most one. Measured: a slab of 40 fp32 tensors of odd sizes (hidden 2575) 487 us without and 460 with such
-// leads, the same of int8 245 and 225, 128 int8 tensors of hidden 2999 1064 and 974 us, a widen of 64
-// M elements 62.2 and 58.1; a block of 128K elements in all is bound by its launch either way. A byte
+// most one. Measured: a slab of 40 fp32 tensors of odd sizes (hidden 2575) 487 us without and 460 with
+// such leads, the same of int8 245 and 225, 128 int8 tensors of hidden 2999 1064 and 974 us, a widen of
+// 64 M elements 62.2 and 58.1; a block of 128K elements in all is bound by its launch either way. A byte
 // copy loses by it, as its loads go off their 16 bytes when its stores come onto them (256 MiB 88
-// us without and 95 with), and zero fill gains nothing. A region whose start is no whole number of elements into the
-// boundary gets none.
+// us without and 95 with), and zero fill gains nothing. A region whose start is no whole number of
+// elements into the boundary gets none.
 constexpr uint64_t kDstAlign = 4096;
 constexpr uint64_t kMinRaggedLead = 1ull << 17;
 uint32_t lead_of(uint32_t kind, uint64_t dst_off, uint64_t numel, bool ragged) {
@@ -92,8 +92,8 @@ struct sh_plan {
 
 namespace {
 
-// build_table in the form that runs fastest, or (fewest) in the one of fewest tiles: no leads that are
-// no whole number of chunks, two tiles to a workgroup of the kinds with fp32 outputs.
+// build_table in the form that runs fastest, or (fewest) in the one that needs fewer workgroups: only
+// leads of whole chunks, two tiles to a workgroup of the kinds with fp32 outputs.
 int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool fewest, std::vector<sh_unpack_desc>& table,
                    sh_plan_info& info, const char* who) {
   if (n > 0 && descs == nullptr) return sh::fail(SH_ERR_INVALID, "%s: descs is NULL", who);
@@ -202,7 +202,7 @@ int build_table_as(const sh_unpack_desc* descs, uint32_t n, bool fewest, std::ve
 
 // Validates the caller's descriptors and produces the launch table (oversize
 // regions split, tiles assigned) and its summary. Host only: no device calls.
-// A table that the fastest form takes past max_tiles is built in the form of fewest tiles.
+// A table that the fastest form takes past max_tiles is built in the other form.
 int build_table(const sh_unpack_desc* descs, uint32_t n, uint32_t max_tiles, std::vector<sh_unpack_desc>& table,
                 sh_plan_info& info, const char* who) {
   const int st = build_table_as(descs, n, false, table, info, who);

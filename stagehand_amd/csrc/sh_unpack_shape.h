@@ -16,8 +16,9 @@ namespace {
 // unrolling and wider chunks each measured 5-25% slower, and so did giving each
 // XCD a contiguous run of tiles (dequant 2%, cast 6%): neighbouring tiles on
 // different XCDs stream faster. Non-temporal accesses help on one side only:
-// the dequant's bf16 stores (+1-1.6%) and the cast's fp32 loads (+1.9%); the
-// other side, or both, measured slower.
+// the stores of the dequants and the widen (bf16 +1-1.6%; fp32 at tile_i8,
+// sh_unpack.hip) and the cast's fp32 loads (+1.9%); the other side, or both,
+// measured slower.
 #ifndef SH_UNPACK_THREADS
 #define SH_UNPACK_THREADS 512
 #endif
@@ -64,7 +65,10 @@ static_assert(kChunkCopy % 16 == 0 && kChunkZero % 16 == 0, "byte chunks are who
 static_assert(kChunkI8 % 4 == 0 && kChunkF32 % 4 == 0, "chunks are whole 32-bit words");
 constexpr uint64_t kMaxDescElems = 1ull << 31;
 
-// Elements that stay together whatever the lead of a short region: a lead is a multiple of this.
+// A lead of a whole number of these is given to any region, in either form of a table (lead_of,
+// build_table, sh_unpack.cpp). For the fp32 outputs it is more than a step of kStepF32: with steps there,
+// regions that start a multiple of 4 but not of 8 or 16 elements off a boundary would gain a lead, and
+// tables near the launch limit that fit now would need a tile more.
 constexpr uint32_t chunk_of(uint32_t kind) {
   return (kind == SH_KIND_I8_ROWSCALE_BF16 || kind == SH_KIND_I8_ROWSCALE_F32) ? kChunkI8
          : kind == SH_KIND_F32_BF16                                              ? kChunkF32

@@ -136,6 +136,8 @@ def test_a_call_waits_for_the_one_before_it_on_another_stream(first, second):
 
 
 def test_captured_call_at_every_replay():
+    """A captured call with a short table shares nothing with other calls: an eager one with a long
+    table (in the scratch array) on a second stream may overlap its replays."""
     descs, sb, db, ns = _table(12)
     src, scales, _z = _inputs(sb, ns, 1)
     got = torch.full((db + 64,), 0xA5, dtype=torch.uint8, device="cuda")
@@ -144,14 +146,20 @@ def test_captured_call_at_every_replay():
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         unpack_noalloc(descs, src, got, scales)
-    other, osb, odb, ons = _table(20)
+    other, osb, odb, ons = _table(40)
     osrc, oscales, _z = _inputs(osb, ons, 2)
+    owant = _want(other, osrc, odb, oscales, None)
+    eager = torch.empty_like(owant)
+    side = torch.cuda.Stream()
     for seed in range(3, 6):
         src.copy_(_inputs(sb, ns, seed)[0])
         got.fill_(0xA5)
+        eager.fill_(0xA5)
         want = _want(descs, src, db, scales, None)
-        graph.replay()
-        eager = torch.empty(odb, dtype=torch.uint8, device="cuda")
-        unpack_noalloc(other, osrc, eager, oscales)  # an eager call between the replays
+        torch.cuda.synchronize()
+        for _ in range(3):
+            graph.replay()
+            unpack_noalloc(other, osrc, eager, oscales, stream=side)
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+        assert torch.equal(eager, owant)

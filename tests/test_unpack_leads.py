@@ -52,11 +52,16 @@ def test_the_other_kinds_get_whole_chunk_leads_only(kind):
         assert tiles(kind, 4096 + lead * width, 64 * per_tile) == 64, lead
 
 
-def test_a_lead_never_refuses_a_table_that_fits_without_it():
+def test_a_ragged_lead_never_refuses_a_table_that_fits_without_it():
     """The largest launch holds (2^32 - 1) // 512 tiles, the allocation-free table 2064384: a region of
-    exactly that many stays accepted from a start whose lead would add one."""
+    exactly that many stays accepted from a start whose lead, no whole number of chunks, would add one.
+    A lead of whole chunks is part of every form of a table: it adds a tile to each of the region's 16
+    pieces of 2^30 elements."""
     max_tiles = (2**32 - 1) // 512
     assert tiles(KIND_F32_BF16, 4096 + 2, 2048, rows=max_tiles) == max_tiles
+    with pytest.raises(ValueError, match="tiles"):
+        tiles(KIND_F32_BF16, 4096 + 64, 2048, rows=max_tiles)
+    assert tiles(KIND_F32_BF16, 4096 + 64, 2048, rows=max_tiles - 16) == max_tiles
     lib = _native.lib()
     for rows, message in ((2064384, b"source"), (2064385, b"tiles")):  # fits: refused for its buffers alone
         table = make_descs([(KIND_F32_BF16, 0, 4098, rows, 2048, 0, 0)])

@@ -1,13 +1,14 @@
 """The allocation-free unpack entry point (``sh_unpack_noalloc``) against the plan-based one.
 
-``sh_unpack_noalloc`` keeps the launch table and tile map in the library's static per-GPU
-scratch instead of device memory ``sh_plan_create`` allocates; the unpack kernels are the same.
-Its output must equal ``sh_unpack`` on the same descriptors and inputs byte for byte. Two calls
-in a row share the scratch: the first is config 2's full dequant (128 descriptors, 270k tiles),
-the second a smaller mixed table whose table and tile map only partly overwrite the first's.
-Calls issued back to back on two streams are ordered on the device (each waits for the previous
-call's kernels before it writes the shared table), so both outputs stay exact. Limits are refused
-with SH_ERR_INVALID before anything is launched.
+``sh_unpack_noalloc`` keeps the launch table and tile map of a table that is too long for one launch's
+arguments (more than 32 regions or 49152 tiles: every table here) in the library's static per-GPU
+scratch instead of device memory ``sh_plan_create`` allocates; the results are the same. Its output
+must equal ``sh_unpack`` on the same descriptors and inputs byte for byte. Two calls in a row share the
+scratch: the first is config 2's full dequant (128 descriptors, 270k tiles), the second a smaller mixed
+table whose table and tile map only partly overwrite the first's. Calls issued back to back on two
+streams are ordered on the device (each waits for the previous call's kernels before it writes the
+shared table), so both outputs stay exact. Limits are refused with SH_ERR_INVALID before anything is
+launched.
 """
 from __future__ import annotations
 
