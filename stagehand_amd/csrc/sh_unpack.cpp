@@ -395,7 +395,7 @@ int launch(const sh_plan* plan, const void* src, size_t src_bytes, const float* 
 // Most tiles of a launch whose table travels in its arguments. The search for a tile's descriptor
 // (five dependent scalar loads, against one of the tile map) costs every workgroup, the table and
 // tile map kernels cost the launch. Measured, arguments against scratch (MI355X, MLP and double-stream
-// blocks): 6 MB 7.2-8.0 against 12.6 us, 100 MB 19.0 and 25.0, 450 MB (18.5K tiles) 67.9 and 74.0, 1 GB
+// blocks): 6 MB 7.0-10.4 against 12.6 us, 100 MB 19.0 and 25.0, 450 MB (18.5K tiles) 67.9 and 74.0, 1 GB
 // (41.5K tiles) 164.3 and 168.2, 1.2 GB (48.7K) 195.8 and 199.6, 1.8 GB (73.8K) 295.1 and 292.8.
 constexpr uint32_t kMaxArgsTiles = 49152;
 

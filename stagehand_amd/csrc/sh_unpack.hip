@@ -653,7 +653,7 @@ __device__ __forceinline__ void unpack_body(const sh_unpack_desc* __restrict__ d
 }
 
 // The launch table in the kernel's arguments: the descriptor of a tile is the last one whose
-// tile_begin is not above it. One launch in place of three: an MLP block of 6 MB 7.2-8.0 us instead of
+// tile_begin is not above it. One launch in place of three: an MLP block of 6 MB 7.0-10.4 us instead of
 // 12.6, bound by the host's call (the rule and both sides are at kMaxArgsTiles, sh_unpack.cpp).
 template <bool HAS_ZP>
 __device__ __forceinline__ void unpack_args_body(const DescArgs& a, const uint8_t* __restrict__ src,
